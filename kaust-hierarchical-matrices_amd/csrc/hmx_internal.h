@@ -143,6 +143,23 @@ struct TLR {
     DBuf<double> diagonal;   // [S*b*b]
 };
 
+// Factor gradients (grad.hip): up to 32 columns of one tile per item, in the
+// level's layout (off: elements from the level's first factor entry).
+struct GradItem {
+    const double *U, *V;
+    int64_t off;
+    int32_t level, m, ncols, rowStart, colStart, pad;
+};
+struct GradPlan {
+    DBuf<GradItem> items;     // tiles of 512 rows and more first
+    int32_t numItems = 0, numTall = 0;
+    int64_t npad = 0;
+    DBuf<int32_t> gmap;       // partial leaves: padded position -> vector index
+    DBuf<double> Xp, Wp;      // padded copies of x and dY (partial leaves, unaligned vectors)
+    uint32_t wsK = 0;
+    bool built = false;
+};
+
 // One level of the hierarchical matrix (src/HMatrix.cuh:9-18).
 struct HLevel {
     int32_t level = 0, numTiles = 0, m = 0, maxRank = 0, capHits = 0;
@@ -345,7 +362,7 @@ struct HMatrix {
     const Structure* structure = nullptr;
     Structure structureCopy;        // owned copy (the caller may free theirs)
     MatvecPlan plan, planT;
-    MatvecPlan gplan, gplanT;        // factor gradients: every tile through z (no dense near-field blocks)
+    GradPlan grad;
     MfPlan mf64, mfMixed;
     // matrix-core plan choices (hmx_hmatrix_set_plan_options)
     int planDenseNear = 1;   // leaf-level tiles of rank > b/2 as dense blocks
@@ -432,10 +449,17 @@ void build_dense_diagonal_padded(Context& c, uint32_t b, uint32_t d, const doubl
                                  double* diag);
 void hmatrix_save(Context& c, const HMatrix& h, const char* path);
 void hmatrix_load(Context& c, const char* path, HMatrix& h);
-void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P, bool denseNear);
+void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P);
+void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const double* X, int64_t ldx, double* Xp);
 PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bool denseNear);
 void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H);
 bool ensure_matvec_ws(MatvecPlan& P, uint32_t K);
+// 16-column blocks (1 to 4) per matrix-core pass of k right-hand sides: the
+// fewest passes of at most 64, all of one width
+inline int mf_pass_blocks(uint32_t k) {
+    const uint32_t passes = (k + 63) / 64;
+    return (int)(((k + passes - 1) / passes + 15) / 16);
+}
 // widest streaming-kernel pass (16, 8, 4 or 1 right-hand sides) for rem columns
 uint32_t pass_width(uint32_t rem);
 void run_matvec_plan(Context& c, MatvecPlan& P, int b, uint32_t k, const double* X, int64_t ldx, double* Y,

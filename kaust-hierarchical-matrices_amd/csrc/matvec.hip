@@ -538,13 +538,16 @@ int row_block(const HMatrix& h) {
     return h.b == 64 && npad >= kRowBlock && npad % kRowBlock == 0 ? kRowBlock : 0;
 }
 
-// denseNear: leaf-level tiles of rank above b/2 as dense blocks (the plans
-// of the products); off for the factor-gradient plans, which need z of
-// every tile
-void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P, bool denseNear) {
+void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const double* X, int64_t ldx, double* Xp) {
+    const int64_t tot = npad * K;
+    k_gather<<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(npad, K, gmap, X, ldx, Xp);
+    HMX_LAUNCHED();
+}
+
+void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P) {
     const int b = (int)h.b, S = (int)h.S;
     HMX_CHECK(h.leafOffsets.size() == (size_t)S + 1, HMX_ESTATE, "H-matrix without leaf offsets");
-    upload_plan(c, P, plan_host(h, transpose, P.chunk, row_block(h), denseNear));
+    upload_plan(c, P, plan_host(h, transpose, P.chunk, row_block(h), h.planDenseNear != 0));
     P.n = h.n;
     P.npad = (int64_t)S * b;
     P.gather = h.n != (uint32_t)P.npad;
@@ -626,8 +629,7 @@ static void run_k(Context& c, const MatvecPlan& P, const MvWork& W, int b, uint3
             continue;
         }
         const int64_t tot = P.npad * K;
-        k_gather<<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(P.npad, K, P.gmap.p, Xs, ldx, W.Xp);
-        HMX_LAUNCHED();
+        gather_padded(c, P.npad, K, P.gmap.p, Xs, ldx, W.Xp);
         run_phases<K>(c, P, W, b, W.Xp, P.npad, W.Yp, ev);
         k_scatter<<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(P.npad, K, P.gmap.p, W.Yp, Ys, ldx);
         HMX_LAUNCHED();
@@ -675,7 +677,7 @@ void hmatvec(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_o
     HMX_CHECK(d_in && d_out, HMX_EINVAL, "null vector pointer");
     HMX_CHECK(d_in != d_out, HMX_EINVAL, "in and out must not alias");
     MatvecPlan& P = transpose ? h.planT : h.plan;
-    if (!P.built) build_matvec_plan(c, h, transpose, P, h.planDenseNear != 0);
+    if (!P.built) build_matvec_plan(c, h, transpose, P);
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     const bool prof = ms != nullptr;
     if (prof)

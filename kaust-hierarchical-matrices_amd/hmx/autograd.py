@@ -81,8 +81,9 @@ class HMatVec(torch.autograd.Function):
         if any(ctx.needs_input_grad[2:]):
             H = op.pipe.H
             nl = H.num_levels - 1
-            dU = {l: torch.zeros_like(op.U[l], requires_grad=False) for l in op.levels}
-            dV = {l: torch.zeros_like(op.V[l], requires_grad=False) for l in op.levels}
+            # the library writes every element
+            dU = {l: torch.empty_like(op.U[l], requires_grad=False) for l in op.levels}
+            dV = {l: torch.empty_like(op.V[l], requires_grad=False) for l in op.levels}
             pu = (ctypes.c_void_p * nl)(*[dU[l].data_ptr() if l in dU else 0 for l in range(1, nl + 1)])
             pv = (ctypes.c_void_p * nl)(*[dV[l].data_ptr() if l in dV else 0 for l in range(1, nl + 1)])
             k = 1 if Xd.dim() == 1 else Xd.shape[0]

@@ -698,7 +698,11 @@ hmx_status hmx_HMatrixVecMultTranspose(hmx_context* ctx, const hmx_hmatrix* h, u
     if (!ctx) return HMX_EINVAL;
     return guard(ctx, [&] {
         NEED(h);
-        hmatvec(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, true, nullptr, 0);
+        // as the forward product: two or more right-hand sides on the matrix cores
+        if (vectorWidth >= 2)
+            hmatvec_multi(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, nullptr, 0, true);
+        else
+            hmatvec(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, true, nullptr, 0);
     });
 }
 
@@ -760,6 +764,7 @@ hmx_status hmx_hmatrix_set_plan_options(hmx_hmatrix* h, int32_t denseNear, int32
     h->planDirectZ = directZ;
     h->planLocality = locality;
     h->mf64 = MfPlan();
+    h->mf64T = MfPlan();
     h->mfMixed = MfPlan();
     h->plan = MatvecPlan();
     h->planT = MatvecPlan();
@@ -770,6 +775,7 @@ hmx_status hmx_hmatrix_set_fp64_layout(hmx_hmatrix* h, int32_t layout) {
     if (!h || layout < 0 || layout > 2) return HMX_EINVAL;
     h->planFp64Layout = layout;
     h->mf64 = MfPlan();
+    h->mf64T = MfPlan();
     return HMX_OK;
 }
 

@@ -278,6 +278,7 @@ void hmatrix_set_level(Context& c, HMatrix& h, int level, const double* U, const
     // plans' dense near-field blocks, are stale now
     ++h.factorGen;
     h.mf64 = MfPlan();
+    h.mf64T = MfPlan();
     h.mfMixed = MfPlan();
     h.plan = MatvecPlan();
     h.planT = MatvecPlan();

@@ -363,7 +363,7 @@ struct HMatrix {
     Structure structureCopy;        // owned copy (the caller may free theirs)
     MatvecPlan plan, planT;
     GradPlan grad;
-    MfPlan mf64, mfMixed;
+    MfPlan mf64, mf64T, mfMixed;
     // matrix-core plan choices (hmx_hmatrix_set_plan_options)
     int planDenseNear = 1;   // leaf-level tiles of rank > b/2 as dense blocks
     int planDirectZ = 1;     // phase 1 stores whole-column z itself (else partials + reduce)
@@ -475,7 +475,8 @@ void hmatvec(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_o
              int iters);
 void dense_rows(Context& c, uint32_t n, uint32_t d, const double* p, const int32_t* perm, double ell, uint32_t nr,
                 const int32_t* rows, uint32_t k, const double* X, double* Y);
-void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters);
+void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters,
+                   bool transpose = false);
 std::vector<int32_t> padding_map(const HMatrix& h, int64_t base);
 bool batch_mf_stale(const Batch& B);
 bool batch_mf_prepare(Context& c, Batch& B, uint32_t k);

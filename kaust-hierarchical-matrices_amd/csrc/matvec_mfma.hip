@@ -1173,22 +1173,27 @@ __global__ void __launch_bounds__(256) k_near_dense(int b, const NearSrc* __rest
 // ---- host side ------------------------------------------------------------------
 namespace {
 
+// A tile as the plan applies it: out rows += U (V^T in rows).  Of the
+// transposed operator, U and V and the two clusters are exchanged.
 struct TileRef {
-    const HLevel* lv;
-    int level, t, r, m;
+    const double *U, *V;  // the tile's first columns, m rows each
+    int r, m;
     uint32_t inCl, outCl;
     int64_t leafBase;  // first leaf of the tile's H-matrix in the plan's leaf space
 };
 
-std::vector<TileRef> all_tiles(const HMatrix& h, int64_t leafBase = 0) {
+std::vector<TileRef> all_tiles(const HMatrix& h, int64_t leafBase = 0, bool transpose = false) {
     std::vector<TileRef> v;
     for (int l = 1; l < h.numLevels; ++l) {
         const HLevel& lv = h.levels[l - 1];
         const auto& tiles = h.structure->tileIndices[l - 1];
         for (int t = 0; t < lv.numTiles; ++t) {
             if (lv.h_ranks[t] == 0) continue;
-            v.push_back(TileRef{&lv, l, t, lv.h_ranks[t], lv.m, compact16((uint32_t)tiles[t]),
-                                compact16((uint32_t)tiles[t] >> 1), leafBase});
+            const double* U = lv.U.p + (size_t)lv.h_offsets[t] * lv.m;
+            const double* V = lv.V.p + (size_t)lv.h_offsets[t] * lv.m;
+            const uint32_t u = compact16((uint32_t)tiles[t]), w = compact16((uint32_t)tiles[t] >> 1);
+            v.push_back(transpose ? TileRef{V, U, lv.h_ranks[t], lv.m, w, u, leafBase}
+                                  : TileRef{U, V, lv.h_ranks[t], lv.m, u, w, leafBase});
         }
     }
     return v;
@@ -1333,12 +1338,11 @@ void build_group(Context& c, const HMatrix& h, int S, bool grouped, MfGroup& G, 
             for (size_t k = i; k < j; ++k) {
                 const int t = ord[k];
                 const TileRef& R = tiles[t].ref;
-                const double* Usrc = R.lv->U.p + (size_t)R.lv->h_offsets[R.t] * m;
                 zb[t] = zcol + (int64_t)(ucols.size() - cd0);
                 for (int q = 0; q < cnt_of(t); ++q) {
                     float fu, fv;
                     scales(t, q, fu, fv);
-                    ucols.push_back(CvCol{Usrc + (size_t)tiles[t].cols[q] * m, 0, m, fu, 0, 0});
+                    ucols.push_back(CvCol{R.U + (size_t)tiles[t].cols[q] * m, 0, m, fu, 0, 0});
                     colScale.push_back(fu * fv * zmul);
                 }
                 for (int q = cnt_of(t); q < cnt_pad(t); ++q) {
@@ -1349,9 +1353,7 @@ void build_group(Context& c, const HMatrix& h, int S, bool grouped, MfGroup& G, 
             for (int q = cntRun; q < rpad; ++q) colScale.push_back(0.f);
             const int64_t leaf0 = row_start(R0) / b;
             if (udirect) {  // one tile, U column-major in place (all its columns, in order)
-                const TileRef& R = R0;
-                add_entries(m, leaf0, MfEntry{nullptr, rpad, (int32_t)zcol, cntRun, m},
-                            R.lv->U.p + (size_t)R.lv->h_offsets[R.t] * m);
+                add_entries(m, leaf0, MfEntry{nullptr, rpad, (int32_t)zcol, cntRun, m}, R0.U);
             } else {
                 for (int r0 = 0; r0 < m; r0 += 32)
                     for (int c0 = 0; c0 < rpad; c0 += 32) trt.push_back(TrTile{cd0, uElems, m, cntRun, rpad, r0, c0, 0});
@@ -1423,11 +1425,10 @@ void build_group(Context& c, const HMatrix& h, int S, bool grouped, MfGroup& G, 
             for (size_t k = i; k < j; ++k) {
                 const int t = ord[k];
                 const TileRef& R = tiles[t].ref;
-                const double* Vsrc = R.lv->V.p + (size_t)R.lv->h_offsets[R.t] * m;
                 for (int q = 0; q < cnt_of(t); ++q) {
                     float fu, fv;
                     scales(t, q, fu, fv);
-                    if (!vdirect) vcol(Vsrc + (size_t)tiles[t].cols[q] * m, fv);
+                    if (!vdirect) vcol(R.V + (size_t)tiles[t].cols[q] * m, fv);
                     else vElems += m;
                     zmap.push_back((int32_t)(zb[t] + q));
                 }
@@ -1441,8 +1442,7 @@ void build_group(Context& c, const HMatrix& h, int S, bool grouped, MfGroup& G, 
             // columns past its last are never read)
             if (vfrag) vElems = v0 + (int64_t)(runCol + 15) / 16 * 16 * m;
             if (vdirect)
-                emit_items(k0, (int64_t)zmap.size(), m, col_start(R0),
-                           (const char*)(R0.lv->V.p + (size_t)R0.lv->h_offsets[R0.t] * m), 0);
+                emit_items(k0, (int64_t)zmap.size(), m, col_start(R0), (const char*)R0.V, 0);
             else
                 emit_items(k0, (int64_t)zmap.size(), m, col_start(R0), nullptr, v0);
             i = j;
@@ -1559,10 +1559,8 @@ void build_near(Context& c, const HMatrix& h, int S, MfPlan& P, const std::vecto
     for (int leaf = 0; leaf < S; ++leaf) {
         ptr[leaf] = (int32_t)src.size();
         for (const TileRef* R : perLeaf[leaf]) {
-            const double* U = R->lv->U.p + (size_t)R->lv->h_offsets[R->t] * R->m;
-            const double* V = R->lv->V.p + (size_t)R->lv->h_offsets[R->t] * R->m;
             colLeaf.push_back((int32_t)(R->leafBase + R->inCl));
-            src.push_back(NearSrc{U, V, (int64_t)src.size() * b * b, R->r, 0});
+            src.push_back(NearSrc{R->U, R->V, (int64_t)src.size() * b * b, R->r, 0});
         }
     }
     ptr[S] = (int32_t)src.size();
@@ -1633,8 +1631,9 @@ void build_near_list(Context& c, const HMatrix& h, int S, MfPlan& P, const std::
 // block-diagonal operator): instance i owns leaves [leafBase_i, leafBase_i +
 // S_i) of one padded leaf space.  Vectors come in as n_i consecutive entries
 // per instance; with partial leaves they are gathered into the padded space
-// and the product scattered back.
-void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P) {
+// and the product scattered back.  transpose: the plan of the transposed
+// operator (U and V exchanged, dense blocks transposed).
+void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P, bool transpose = false) {
     HMX_CHECK(!hs.empty(), HMX_EINVAL, "empty plan set");
     const HMatrix& h0 = *hs[0];
     check_bucket(h0);
@@ -1646,7 +1645,7 @@ void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P)
     for (HMatrix* h : hs) {
         HMX_CHECK(h->b == (uint32_t)b, HMX_EINVAL, "all instances of a batch need the same bucketSize");
         HMX_CHECK(h->leafOffsets.size() == (size_t)h->S + 1, HMX_ESTATE, "H-matrix without leaf offsets");
-        std::vector<TileRef> t = all_tiles(*h, leafBase);
+        std::vector<TileRef> t = all_tiles(*h, leafBase, transpose);
         all.insert(all.end(), t.begin(), t.end());
         std::vector<int32_t> g = padding_map(*h, vecBase);
         gm.insert(gm.end(), g.begin(), g.end());
@@ -1690,9 +1689,14 @@ void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P)
     int64_t off = 0;
     for (HMatrix* h : hs) {
         const int64_t e = (int64_t)h->S * b * b;
-        k_diag_rowmajor<double><<<(unsigned)((e + 255) / 256), 256, 0, c.stream>>>(e, b, h->diag.p,
-                                                                                  (double*)P.Drm.p + off);
-        HMX_LAUNCHED();
+        if (transpose) {  // column-major blocks are their transposes' row-major form
+            HMX_HIP(hipMemcpyAsync((double*)P.Drm.p + off, h->diag.p, (size_t)e * sizeof(double),
+                                   hipMemcpyDeviceToDevice, c.stream));
+        } else {
+            k_diag_rowmajor<double><<<(unsigned)((e + 255) / 256), 256, 0, c.stream>>>(e, b, h->diag.p,
+                                                                                      (double*)P.Drm.p + off);
+            HMX_LAUNCHED();
+        }
         off += e;
     }
     HMX_HIP(hipStreamSynchronize(c.stream));
@@ -1948,11 +1952,14 @@ void run_fp64_plan(Context& c, MfPlan& P, uint32_t k, const double* d_in, double
     }
 }
 
-void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters) {
+// transpose: H^T, through a plan of its own (N = 65536 2D, 32 right-hand
+// sides: 0.61 ms; the streaming kernels, 16 wide, took 1.9)
+void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters,
+                   bool transpose) {
     HMX_CHECK(k >= 1, HMX_EINVAL, "multi-RHS matvec: vectorWidth must be >= 1");
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
-    if (!h.mf64.built) build_fp64_plan_set(c, {&h}, h.mf64);
-    MfPlan& P = h.mf64;
+    MfPlan& P = transpose ? h.mf64T : h.mf64;
+    if (!P.built) build_fp64_plan_set(c, {&h}, P, transpose);
     ensure_fp64_ws(c, P, (k % 64 == 0) ? 64 : 16);
     Events ev;
     if (ms) ev.create();
@@ -2018,9 +2025,7 @@ void hmatrix_make_mixed(Context& c, HMatrix& h, double target) {
     }
     for (const TileRef& R : tiles) {
         colBase.push_back((int64_t)cd.size());
-        const double* U = R.lv->U.p + (size_t)R.lv->h_offsets[R.t] * R.m;
-        const double* V = R.lv->V.p + (size_t)R.lv->h_offsets[R.t] * R.m;
-        for (int j = 0; j < R.r; ++j) cd.push_back(ColDesc{U + (size_t)j * R.m, V + (size_t)j * R.m, R.m, 0});
+        for (int j = 0; j < R.r; ++j) cd.push_back(ColDesc{R.U + (size_t)j * R.m, R.V + (size_t)j * R.m, R.m, 0});
     }
     const int64_t nc = (int64_t)cd.size();
     std::vector<double> v2(nc), um(nc), vm(nc);

@@ -263,7 +263,7 @@ hmx_status hmx_freeHMatrix(hmx_hmatrix* h);
    reference needs n = S*b, src/cutlassDiagonalXVector.cu:59-65) the vectors
    are gathered into the padded leaf space and the product scattered back.
    One right-hand side runs the FP64 streaming kernels, two or more the FP64
-   matrix cores (passes of 16, or 64 when vectorWidth is a multiple of 64). */
+   matrix cores (passes of 16, 32, 48 or 64, all of a call of one width). */
 hmx_status hmx_HMatrixVecMult(hmx_context* ctx, const hmx_hmatrix* h, uint32_t vectorWidth, const double* d_in,
                               double* d_out);
 /* No counterpart in the reference: for callers that cannot allocate device
@@ -280,8 +280,8 @@ hmx_status hmx_HMatrixVecMult(hmx_context* ctx, const hmx_hmatrix* h, uint32_t v
 hmx_status hmx_HMatrixVecMultNoAlloc(hmx_context* ctx, const hmx_hmatrix* h, uint32_t vectorWidth,
                                      const double* d_in, double* d_out);
 /* out = H^T * in (no reference counterpart; the backward of HMatrixVecMult);
-   any vectorWidth >= 1 and any n, on the streaming kernels in passes of 16,
-   8, 4 or 1 right-hand sides */
+   any vectorWidth >= 1 and any n: one right-hand side on the streaming
+   kernels, two or more on the matrix cores as hmx_HMatrixVecMult. */
 hmx_status hmx_HMatrixVecMultTranspose(hmx_context* ctx, const hmx_hmatrix* h, uint32_t vectorWidth,
                                        const double* d_in, double* d_out);
 /* Times the matvec kernels with hipEvents on the context stream over iters
@@ -413,7 +413,7 @@ hmx_status hmx_generateHMatrixDirectBatch(hmx_context* ctx, int32_t count, const
 hmx_status hmx_batch_create(hmx_context* ctx, int32_t count, hmx_hmatrix* const* hmatrices, hmx_batch** batch);
 hmx_status hmx_batch_info(const hmx_batch* batch, int64_t* totalPoints, int64_t* totalLeaves, int32_t* chunk);
 /* FP64, any vectorWidth >= 1 (two or more run on the matrix cores, in passes
-   of 16 or 64 columns).  useGraph != 0: the launch
+   of 16, 32, 48 or 64 columns).  useGraph != 0: the launch
    sequence is captured in a hipGraph on first use (again when d_in, d_out or
    vectorWidth change) and replayed, ordered after prior work on the context
    stream. */

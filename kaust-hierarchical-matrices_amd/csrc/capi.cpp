@@ -575,7 +575,7 @@ hmx_status hmx_HMatrixVecMult(hmx_context* ctx, const hmx_hmatrix* h, uint32_t v
     return guard(ctx, [&] {
         NEED(h);
         // two or more right-hand sides: the FP64 matrix cores (passes of 16
-        // or 64, partial leaves through the padded space); one: the
+        // to 64, partial leaves through the padded space); one: the
         // streaming kernels
         if (vectorWidth >= 2)
             hmatvec_multi(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, nullptr, 0);

@@ -455,7 +455,11 @@ PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bo
 void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H);
 bool ensure_matvec_ws(MatvecPlan& P, uint32_t K);
 // 16-column blocks (1 to 4) per matrix-core pass of k right-hand sides: the
-// fewest passes of at most 64, all of one width
+// fewest passes of at most 64, all of one width (z's layout depends on it).
+// Every pass reads all factors, so one of 32 beats two of 16 (N = 60000 3D:
+// FP64 1.53 against 2.41 ms, mixed 0.46 against 0.81), one of 48 three (2.04
+// against 3.63; 0.52 against 1.21) and one of 64 four even for 50 right-hand
+// sides (2.45 against 4.81; 0.57 against 1.61).
 inline int mf_pass_blocks(uint32_t k) {
     const uint32_t passes = (k + 63) / 64;
     return (int)(((k + passes - 1) / passes + 15) / 16);

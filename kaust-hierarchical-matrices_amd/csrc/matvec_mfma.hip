@@ -1,5 +1,5 @@
 // Multi right-hand-side H-matvec on the matrix cores, FP64 (any number of
-// right-hand sides, in passes of 16 or 64) and mixed FP32/FP16 (16 or 64).
+// right-hand sides) and mixed FP32/FP16, in passes of 16, 32, 48 or 64.
 //
 //   phase 1  Z = V^T X per tile: one wave per (tile, 64 columns, 1024 rows),
 //            D(16 cols x 16 rhs) += A(16 cols x K rows) B(K rows x 16 rhs);
@@ -195,10 +195,10 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     // (readfirstlane), the item loads into scalar registers and the loop runs
     // without exec masks: FP32/FP16 phase 1 8.3 -> 8.0 ms at N = 2^20, 64
     // right-hand sides; FP64 with 16 (256-cloud batch) 19.15 -> 18.95 ms per
-    // call.  The FP64 kernel with 64 is scheduled worse that way (36.4 ->
-    // 40.7 ms, measured) and keeps the per-lane index.
+    // call.  The FP64 kernels with 48 and 64 are scheduled worse that way (64:
+    // 36.4 -> 40.7 ms, measured) and keep the per-lane index.
     const int wv = wg * 4 + (int)(threadIdx.x >> 6);
-    const int wid = (sizeof(T) < 8 || NB == 1) ? __builtin_amdgcn_readfirstlane(wv) : wv;
+    const int wid = (sizeof(T) < 8 || NB <= 2) ? __builtin_amdgcn_readfirstlane(wv) : wv;
     if (wid >= nItems) return;
     const int lg = lane >> 4, lc = lane & 15;
     using ACC = typename M::acc_t;
@@ -209,14 +209,15 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     for (int g = 0; g < CG; ++g)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[g][nb] = typename M::accv{0, 0, 0, 0};
-    // FP64 with 64 right-hand sides and FP16: software pipelined, the
+    // FP64 with 48 or 64 right-hand sides and FP16: software pipelined, the
     // operands of super-step r0 + 16*KL are in flight while the MFMAs of
     // super-step r0 run (FP64 36.4 ms vs 39.1 without, at N = 2^20; FP16
-    // 4.4 -> 4.2 ms with the fragment-ordered copies).  FP64 with 16 and
-    // FP32: no register double buffer -- the registers it frees buy more
-    // waves per SIMD, which hide the load latency better (FP64 16 RHS 16.6 ->
-    // 15.9 ms; FP32 slower with it).
-    constexpr bool PF = !SPLIT && ((sizeof(T) == 8 && NB > 1) || sizeof(T) == 2);
+    // 4.4 -> 4.2 ms with the fragment-ordered copies).  FP64 with 16 or
+    // 32 and FP32: no register double buffer -- the registers it frees buy
+    // more waves per SIMD, which hide the load latency better (FP64 16 RHS
+    // 16.6 -> 15.9 ms; 32 RHS at N = 60000 3D, whole call 1621 -> 1529 us;
+    // FP32 slower with it).
+    constexpr bool PF = !SPLIT && ((sizeof(T) == 8 && NB > 2) || sizeof(T) == 2);
     T a[CG][VL], bx[NB][VL], an[CG][VL], bn[NB][VL];
     constexpr int E16 = 16 / (int)sizeof(T), NP = VL / E16;
     auto load = [&](int r0, T (&A)[CG][VL], T (&B)[NB][VL]) {
@@ -1705,6 +1706,17 @@ void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P,
     P.built = true;
 }
 
+// f(NB as a constant) for passes of NB = 1 to 4 blocks of 16 right-hand sides
+template <class F>
+void with_blocks(int NB, F&& f) {
+    switch (NB) {
+        case 1: f(std::integral_constant<int, 1>{}); break;
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 3: f(std::integral_constant<int, 3>{}); break;
+        default: f(std::integral_constant<int, 4>{}); break;
+    }
+}
+
 // zLoOff >= 0 (T = FP16): z as FP16 hi + lo, lo at zLoOff
 template <class ACC, class T>
 void reduce_group(Context& c, MfGroup& G, int NR, const float* rhsScale = nullptr, int64_t zLoOff = -1) {
@@ -1715,16 +1727,16 @@ void reduce_group(Context& c, MfGroup& G, int NR, const float* rhsScale = nullpt
         k<<<blocks, 256, 0, c.stream>>>(G.numRed, G.numColsPad, G.redCol.p, G.colPart.p, G.colNpart.p, cs,
                                         (const ACC*)G.zpart.p, (T*)G.zt.p, rhsScale, zLoOff);
     };
-    if constexpr (sizeof(T) == 2) {
-        if (zLoOff >= 0) {
-            if (NR == 64) launch(k_mf_reduce<T, ACC, 64, true>);
-            else launch(k_mf_reduce<T, ACC, 16, true>);
-            HMX_LAUNCHED();
-            return;
+    with_blocks(NR / 16, [&](auto nb) {
+        constexpr int R = 16 * decltype(nb)::value;
+        if constexpr (sizeof(T) == 2) {
+            if (zLoOff >= 0) {
+                launch(k_mf_reduce<T, ACC, R, true>);
+                return;
+            }
         }
-    }
-    if (NR == 64) launch(k_mf_reduce<T, ACC, 64>);
-    else launch(k_mf_reduce<T, ACC, 16>);
+        launch(k_mf_reduce<T, ACC, R>);
+    });
     HMX_LAUNCHED();
 }
 
@@ -1939,28 +1951,27 @@ bool ensure_fp64_ws(Context& c, MfPlan& P, int NR) {
     return changed;
 }
 
-// Y = H X for k right-hand sides (ld = the plan's n) in passes of 64 (k a
-// multiple of 64) or 16, the last pass padded with zero columns
+// Y = H X for k right-hand sides (ld = the plan's n) in passes of
+// mf_pass_blocks(k) * 16, the last pass padded with zero columns
 void run_fp64_plan(Context& c, MfPlan& P, uint32_t k, const double* d_in, double* d_out, Events& ev) {
-    const int NB = (k % 64 == 0) ? 4 : 1, NR = 16 * NB;
+    const int NB = mf_pass_blocks(k), NR = 16 * NB;
     for (uint32_t s0 = 0; s0 < k; s0 += NR) {
         const int kk = (int)std::min<uint32_t>(NR, k - s0);
         const double* X = d_in + (size_t)s0 * P.n;
         double* Y = d_out + (size_t)s0 * P.n;
-        if (NB == 4) run_fp64<4>(c, P, X, P.n, kk, Y, P.n, ev);
-        else run_fp64<1>(c, P, X, P.n, kk, Y, P.n, ev);
+        with_blocks(NB, [&](auto nb) { run_fp64<decltype(nb)::value>(c, P, X, P.n, kk, Y, P.n, ev); });
     }
 }
 
 // transpose: H^T, through a plan of its own (N = 65536 2D, 32 right-hand
-// sides: 0.61 ms; the streaming kernels, 16 wide, took 1.9)
+// sides: 0.37 ms; the streaming kernels, 16 wide, took 1.9)
 void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters,
                    bool transpose) {
     HMX_CHECK(k >= 1, HMX_EINVAL, "multi-RHS matvec: vectorWidth must be >= 1");
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = transpose ? h.mf64T : h.mf64;
     if (!P.built) build_fp64_plan_set(c, {&h}, P, transpose);
-    ensure_fp64_ws(c, P, (k % 64 == 0) ? 64 : 16);
+    ensure_fp64_ws(c, P, 16 * mf_pass_blocks(k));
     Events ev;
     if (ms) ev.create();
     const int reps = ms ? std::max(1, iters) : 1;
@@ -1996,7 +2007,7 @@ bool batch_mf_prepare(Context& c, Batch& B, uint32_t k) {
         for (const HMatrix* h : B.hs) B.mfGen.push_back(h->factorGen);
         changed = true;
     }
-    return ensure_fp64_ws(c, B.mf, (k % 64 == 0) ? 64 : 16) || changed;
+    return ensure_fp64_ws(c, B.mf, 16 * mf_pass_blocks(k)) || changed;
 }
 
 void batch_mf_run(Context& c, Batch& B, uint32_t k, const double* d_in, double* d_out) {
@@ -2239,14 +2250,14 @@ bool ensure_mixed_ws(Context& c, MfPlan& P, int NR) {
     return changed;
 }
 
-// Y = H X for any k >= 1 (FP32, ld n): passes of 64 (k a multiple of 64) or
-// 16, the last one padded with zero columns
+// Y = H X for any k >= 1 (FP32, ld n) in passes of mf_pass_blocks(k) * 16,
+// the last one padded with zero columns
 void hmatvec_mixed(Context& c, HMatrix& h, uint32_t k, const float* d_in, float* d_out, float* ms, int iters) {
     HMX_CHECK(h.mfMixed.built, HMX_ESTATE, "mixed-precision factors not built (call hmx_hmatrix_make_mixed)");
     HMX_CHECK(k >= 1, HMX_EINVAL, "mixed matvec: vectorWidth must be >= 1");
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = h.mfMixed;
-    const int NB = (k % 64 == 0) ? 4 : 1;
+    const int NB = mf_pass_blocks(k);
     const int NR = 16 * NB;
     ensure_mixed_ws(c, P, NR);
     Events ev;
@@ -2258,8 +2269,7 @@ void hmatvec_mixed(Context& c, HMatrix& h, uint32_t k, const float* d_in, float*
             const int kk = (int)std::min<uint32_t>(NR, k - s0);
             const float* X = d_in + (size_t)s0 * h.n;
             float* Y = d_out + (size_t)s0 * h.n;
-            if (NB == 4) run_mixed<4>(c, P, X, h.n, kk, Y, h.n, ev);
-            else run_mixed<1>(c, P, X, h.n, kk, Y, h.n, ev);
+            with_blocks(NB, [&](auto nb) { run_mixed<decltype(nb)::value>(c, P, X, h.n, kk, Y, h.n, ev); });
         }
         finish_timing(ev, acc);
     }

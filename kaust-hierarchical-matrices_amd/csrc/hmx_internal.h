@@ -195,6 +195,12 @@ struct NearRef {
     int32_t r, outLeaf, inLeaf, pad;
 };
 
+// The factors of a dense block A B^T, r columns of b rows each (near_blocks)
+struct NearPair {
+    const double *A, *B;
+    int32_t r, pad;
+};
+
 // Host form of a matvec plan over the padded vector space (position
 // leaf*b + i for point i of a leaf; padded positions hold zeros).
 struct PlanHost {
@@ -453,6 +459,8 @@ void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P);
 void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const double* X, int64_t ldx, double* Xp);
 PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bool denseNear);
 void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H);
+// out[q] = A_q B_q^T, row-major b x b blocks one after the other
+void near_blocks_f64(Context& c, int b, int64_t n, const NearPair* src, double* out);
 bool ensure_matvec_ws(MatvecPlan& P, uint32_t K);
 // 16-column blocks (1 to 4) per matrix-core pass of k right-hand sides: the
 // fewest passes of at most 64, all of one width (z's layout depends on it).

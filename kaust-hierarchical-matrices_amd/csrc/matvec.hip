@@ -359,19 +359,6 @@ __global__ void __launch_bounds__(256) k_transpose_blocks(int S, int b, const do
     DT[leaf * per + (int64_t)q * b + c] = D[e];
 }
 
-// dense near-field blocks, column-major: out[q][col*b + row] = sum_a U[a*b + row] V[a*b + col]
-__global__ void __launch_bounds__(256) k_near_dense_cm(int b, const NearRef* __restrict__ src,
-                                                       double* __restrict__ out) {
-    const NearRef t = src[blockIdx.x];
-    double* o = out + (size_t)blockIdx.x * b * b;
-    for (int e = threadIdx.x; e < b * b; e += 256) {
-        const int col = e / b, row = e % b;
-        double v = 0.0;
-        for (int a = 0; a < t.r; ++a) v = fma(t.U[(size_t)a * b + row], t.V[(size_t)a * b + col], v);
-        o[e] = v;
-    }
-}
-
 // vectors (ldx apart) <-> the padded space (npad apart), K right-hand sides
 __global__ void __launch_bounds__(256) k_gather(int64_t npad, int K, const int32_t* __restrict__ gmap,
                                                 const double* __restrict__ X, int64_t ldx, double* __restrict__ Xp) {
@@ -506,10 +493,12 @@ void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H) {
     put(c, P.nearCol, col);
     P.nearD.alloc((size_t)std::max<int64_t>(1, P.numNear) * b * b);
     if (P.numNear) {
-        DBuf<NearRef> d_src;
-        put(c, d_src, nears);
-        k_near_dense_cm<<<(unsigned)P.numNear, 256, 0, c.stream>>>(b, d_src.p, P.nearD.p);
-        HMX_LAUNCHED();
+        std::vector<NearPair> pairs;  // V first: column-major blocks
+        pairs.reserve(nears.size());
+        for (const NearRef& nr : nears) pairs.push_back(NearPair{nr.V, nr.U, nr.r, 0});
+        DBuf<NearPair> d_src;
+        put(c, d_src, pairs);
+        near_blocks_f64(c, b, P.numNear, d_src.p, P.nearD.p);
         HMX_HIP(hipStreamSynchronize(c.stream));
     }
     P.bytes = H.lowRankBytes + 8ull * (uint64_t)(S + P.numNear) * b * b;

@@ -93,11 +93,13 @@ hmx_status hmx_create(hmx_context** ctx, void* stream) {
         delete c;
         return st;
     }
+    pool_context_created();
     *ctx = c;
     return HMX_OK;
 }
 
 hmx_status hmx_destroy(hmx_context* ctx) {
+    if (ctx) pool_context_destroyed();
     delete ctx;
     return HMX_OK;
 }

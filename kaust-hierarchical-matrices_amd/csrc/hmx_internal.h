@@ -46,7 +46,15 @@ inline void alloc_fault_point() {
         throw Error(HMX_ENOMEM, "forced device allocation failure (allocation " + std::to_string(k) + ")");
 }
 
-// Owning device buffer (hipMalloc / hipFree), movable, not copyable.
+// Device memory of the library (pool.cpp): freed blocks are kept, within a
+// bound, for the next allocations
+void* pool_alloc(size_t bytes);
+void pool_free(void* p);
+size_t pool_held_bytes();  // held on the current device
+void pool_context_created();
+void pool_context_destroyed();  // the last one gives everything held back
+
+// Owning device buffer, movable, not copyable.
 template <class T>
 struct DBuf {
     T* p = nullptr;
@@ -81,7 +89,7 @@ struct DBuf {
         release();
         if (count) {
             alloc_fault_point();
-            HMX_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+            p = static_cast<T*>(pool_alloc(count * sizeof(T)));
             g_liveBytes.fetch_add((int64_t)(count * sizeof(T)));
         }
         n = count;
@@ -90,7 +98,7 @@ struct DBuf {
         if (keep) {
             keep.reset();
         } else if (p) {
-            (void)hipFree(p);
+            pool_free(p);
             g_liveBytes.fetch_sub((int64_t)(n * sizeof(T)));
         }
         p = nullptr;

@@ -1718,7 +1718,7 @@ void build_fp64_plan_set(Context& c, const std::vector<HMatrix*>& hs, MfPlan& P,
         for (const GroupTile& gt : tiles) est += 2ull * (uint64_t)(gt.ref.r + kPad) * gt.ref.m * sizeof(double);
         size_t fr = 0, totMem = 0;
         HMX_HIP(hipMemGetInfo(&fr, &totMem));
-        copy = est <= fr / 2;
+        copy = est <= (fr + pool_held_bytes()) / 2;
     }
     P.ucm = !copy;
     build_group(c, h0, S, grouped, P.g[0], 0, tiles, P.ucm, nullptr, nullptr, nullptr);

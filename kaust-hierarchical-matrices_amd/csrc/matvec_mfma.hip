@@ -160,6 +160,17 @@ __device__ inline size_t xb_index(int64_t row, int s, int sh) {
     return ((((size_t)(row >> sh)) * NR + (size_t)s) << sh) + (size_t)(row & ((1 << sh) - 1));
 }
 
+// Steps whose operands are in flight at once with 16 right-hand sides, in
+// registers, while earlier ones are multiplied.  A step is short then (8
+// products a wave in FP64 phase 2) against the latency of its loads, and the
+// registers are there: FP64 phase 2 of 48 clouds (13 GB) 2193 -> 2036 us with
+// 4 steps instead of 2, whole calls of 16 at N = 60000 3D 1210 -> 1020 us,
+// mixed phase 2 at N = 65536 2D 67 -> 60.  FP64 phase 1 gains from 2 steps (no
+// copies between the buffers) and not from 3 or 4; FP16 phase 1 keeps its
+// double buffer (29.6 against 32.9 us with 4).
+constexpr int kPipe = 4;   // phase 2
+constexpr int kPipe1 = 2;  // phase 1
+
 // ---- phase 1 ---------------------------------------------------------------
 // SPLIT (T = FP16): the FP32 group of a mixed plan with V held as FP16 hi +
 // lo (V/scale = hi + lo, lo at V + vLoOff) and the right-hand sides as FP16
@@ -198,11 +209,14 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     // call.  The FP64 kernels with 48 and 64 are scheduled worse that way (64:
     // 36.4 -> 40.7 ms, measured) and keep the per-lane index.
     const int wv = wg * 4 + (int)(threadIdx.x >> 6);
-    const int wid = (sizeof(T) < 8 || NB <= 2) ? __builtin_amdgcn_readfirstlane(wv) : wv;
+    const int unit = (sizeof(T) < 8 || NB <= 2) ? __builtin_amdgcn_readfirstlane(wv) : wv;
+    constexpr int UPI = kMfCols / 16 / CG;  // waves per item, CG 16-column groups each
+    const int wid = unit / UPI, g0 = UPI > 1 ? (unit % UPI) * CG : 0;
     if (wid >= nItems) return;
     const int lg = lane >> 4, lc = lane & 15;
     using ACC = typename M::acc_t;
     const MfItem it = items[wid];
+    if (16 * g0 >= it.ncols) return;
     const T* __restrict__ V = (const T*)it.v;
     typename M::accv acc[CG][NB];
 #pragma unroll
@@ -217,7 +231,8 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     // more waves per SIMD, which hide the load latency better (FP64 16 RHS
     // 16.6 -> 15.9 ms; 32 RHS at N = 60000 3D, whole call 1621 -> 1529 us;
     // FP32 slower with it).
-    constexpr bool PF = !SPLIT && ((sizeof(T) == 8 && NB > 2) || sizeof(T) == 2);
+    constexpr bool DEEP = sizeof(T) == 8 && NB == 1;
+    constexpr bool PF = !DEEP && !SPLIT && ((sizeof(T) == 8 && NB > 2) || sizeof(T) == 2);
     T a[CG][VL], bx[NB][VL], an[CG][VL], bn[NB][VL];
     constexpr int E16 = 16 / (int)sizeof(T), NP = VL / E16;
     auto load = [&](int r0, T (&A)[CG][VL], T (&B)[NB][VL]) {
@@ -229,8 +244,8 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
             const int pstride = 16 * E16 * (min(16 * KL, it.rows - r0) / VL);
 #pragma unroll
             for (int g = 0; g < CG; ++g) {
-                if (rok && 16 * g + lc < it.ncols) {
-                    const T* vp = V + (size_t)g * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
+                if (rok && 16 * (g0 + g) + lc < it.ncols) {
+                    const T* vp = V + (size_t)(g0 + g) * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
 #pragma unroll
                     for (int p = 0; p < NP; ++p) vload16_nt(vp + p * pstride, &A[g][p * E16]);
                 } else {
@@ -253,8 +268,8 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
             const int pstride = 16 * E16 * (min(16 * KL, it.rows - r0) / VL);
 #pragma unroll
             for (int g = 0; g < CG; ++g) {
-                if (rok && 16 * g + lc < it.ncols) {
-                    const T* vp = V + (size_t)g * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
+                if (rok && 16 * (g0 + g) + lc < it.ncols) {
+                    const T* vp = V + (size_t)(g0 + g) * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
 #pragma unroll
                     for (int p = 0; p < NP; ++p) vload16_nt(vp + p * pstride, &A[g][p * E16]);
                 } else {
@@ -274,7 +289,7 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
         } else {
 #pragma unroll
             for (int g = 0; g < CG; ++g) {
-                const int col = 16 * g + lc;
+                const int col = 16 * (g0 + g) + lc;
                 if (rok && col < it.ncols) vload_f(V + (size_t)col * it.ld + rr, A[g]);
                 else vzero(A[g]);
             }
@@ -296,8 +311,8 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
         const int pstride = 16 * E16 * (min(16 * KL, it.rows - r0) / VL);
 #pragma unroll
         for (int g = 0; g < CG; ++g) {
-            if (rok && 16 * g + lc < it.ncols) {
-                const T* vp = V + vLoOff + (size_t)g * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
+            if (rok && 16 * (g0 + g) + lc < it.ncols) {
+                const T* vp = V + vLoOff + (size_t)(g0 + g) * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
 #pragma unroll
                 for (int p = 0; p < NP; ++p) vload16_nt(vp + p * pstride, &A[g][p * E16]);
             } else {
@@ -315,8 +330,28 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
             }
         }
     };
+    if constexpr (DEEP) {
+        constexpr int SS = 16 * KL;
+        T pa[kPipe1][CG][VL], pb[kPipe1][NB][VL];
+#pragma unroll
+        for (int d = 0; d < kPipe1; ++d)
+            if (d * SS < it.rows) load(d * SS, pa[d], pb[d]);
+        for (int r0 = 0; r0 < it.rows; r0 += kPipe1 * SS)
+#pragma unroll
+            for (int d = 0; d < kPipe1; ++d) {
+                const int r = r0 + d * SS;
+                if (r < it.rows) {
+#pragma unroll
+                    for (int e = 0; e < VL / MX::KL; ++e)
+#pragma unroll
+                        for (int g = 0; g < CG; ++g)
+                            acc[g][0] = MX::op(MX::make(&pa[d][g][e * MX::KL]), MX::make(&pb[d][0][e * MX::KL]), acc[g][0]);
+                    if (r + kPipe1 * SS < it.rows) load(r + kPipe1 * SS, pa[d], pb[d]);
+                }
+            }
+    }
     if (PF) load(0, a, bx);
-    for (int r0 = 0; r0 < it.rows; r0 += 16 * KL) {
+    for (int r0 = 0; !DEEP && r0 < it.rows; r0 += 16 * KL) {
         const bool more = PF && r0 + 16 * KL < it.rows;
         if (!PF) load(r0, a, bx);
         if constexpr (SPLIT) load_lo(r0, an, bn);
@@ -366,7 +401,7 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
             typedef TZ tv4 __attribute__((ext_vector_type(4)));
 #pragma unroll
             for (int g = 0; g < CG; ++g) {
-                const int col0 = 16 * g + 4 * lg;
+                const int col0 = 16 * (g0 + g) + 4 * lg;
                 if (col0 >= it.ncols) continue;
                 const int64_t zc = zmap[it.zidx + col0];
                 ACC cs[4] = {(ACC)1, (ACC)1, (ACC)1, (ACC)1};
@@ -405,7 +440,7 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
         for (int g = 0; g < CG; ++g)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int col = 16 * g + M::out_row(lg, v);
+                const int col = 16 * (g0 + g) + M::out_row(lg, v);
                 if (col < it.ncols) {
                     // column scale by V order: no load waits on the z-column map
                     const int64_t zc = zmap[it.zidx + col];
@@ -421,7 +456,7 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     for (int g = 0; g < CG; ++g)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int col = 16 * g + M::out_row(lg, v);
+            const int col = 16 * (g0 + g) + M::out_row(lg, v);
             if (col < it.ncols)
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
@@ -476,13 +511,12 @@ __global__ void __launch_bounds__(256) k_mf_reduce(int64_t nred, int64_t ldz, co
 // acc[rg][nb] += U[16rg.., cols] Z[cols, rhs 16nb..].  The operands of the
 // next 16*KL-column step (possibly of the next entry) load while the current
 // step's MFMAs run.  rowOff: the wave's first row inside the entries' U.
-template <int BL, bool UCM, class T, int NB>
+template <int RG, bool UCM, class T, int NB>
 __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1, const T* __restrict__ Z, int rowOff,
-                               int lg, int lc, int kvalid, typename Mfma<T>::accv (&acc)[BL / 16][NB]) {
+                               int lg, int lc, int kvalid, typename Mfma<T>::accv (&acc)[RG][NB]) {
     using M = Mfma<T>;
     using MX = typename std::conditional<std::is_same<T, _Float16>::value, Mfma32h, M>::type;  // as in phase 1
-    constexpr int KL = M::KL, VL = 4 * KL, SS = 16 * KL, NR = 16 * NB, RG = BL / 16, E16 = 16 / (int)sizeof(T),
-                  NP = VL / E16;
+    constexpr int KL = M::KL, VL = 4 * KL, SS = 16 * KL, NR = 16 * NB, E16 = 16 / (int)sizeof(T), NP = VL / E16;
     if (e0 >= e1) return;
     T a[RG][VL], bz[NB][VL], an[RG][VL], bn[NB][VL];
     auto load = [&](const MfEntry& en, int c0, T (&A)[RG][VL], T (&B)[NB][VL]) {
@@ -528,6 +562,41 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
             for (int nb = 0; nb < NB; ++nb) vzero(B[nb]);
         }
     };
+    if constexpr (NB == 1) {
+        // kPipe steps of the list in flight; the next entry's descriptor is
+        // read an entry ahead
+        T pa[kPipe][RG][VL], pb[kPipe][NB][VL];
+        int e = e0, c0 = 0;
+        MfEntry en = ents[e], nx = ents[min(e + 1, e1 - 1)];
+        bool full[kPipe];
+        auto fill = [&](int d) {
+            full[d] = e < e1;
+            if (full[d]) {
+                load(en, c0, pa[d], pb[d]);
+                c0 += SS;
+                if (c0 >= en.rpad) {
+                    c0 = 0;
+                    ++e;
+                    en = nx;
+                    nx = ents[min(e + 1, e1 - 1)];
+                }
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < kPipe; ++d) fill(d);
+        while (full[0])
+#pragma unroll
+            for (int d = 0; d < kPipe; ++d)
+                if (full[d]) {
+#pragma unroll
+                    for (int q = 0; q < VL / MX::KL; ++q)
+#pragma unroll
+                        for (int rg = 0; rg < RG; ++rg)
+                            acc[rg][0] = MX::op(MX::make(&pa[d][rg][q * MX::KL]), MX::make(&pb[d][0][q * MX::KL]), acc[rg][0]);
+                    fill(d);
+                }
+        return;
+    }
     int e = e0, c0 = 0;
     MfEntry en = ents[e];
     load(en, 0, a, bz);
@@ -568,13 +637,13 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
 // FP16 group), three FP16 16x16x32 products per step (hi*hi + hi*lo +
 // lo*hi).  No register double buffer: the two operand sets take the
 // registers a prefetch would.
-template <int BL, int NB>
+template <int RG, int NB>
 __device__ inline void lr_rows_split(const MfEntry* __restrict__ ents, int e0, int e1, const _Float16* __restrict__ Z,
                                      int64_t zLoOff, int64_t uLoOff, int rowOff, int lg, int lc, int kvalid,
-                                     v4f (&acc)[BL / 16][NB]) {
+                                     v4f (&acc)[RG][NB]) {
     using M = Mfma<_Float16>;
     using MX = Mfma32h;
-    constexpr int KL = M::KL, VL = 4 * KL, SS = 16 * KL, NR = 16 * NB, RG = BL / 16, E16 = 8, NP = VL / E16,
+    constexpr int KL = M::KL, VL = 4 * KL, SS = 16 * KL, NR = 16 * NB, E16 = 8, NP = VL / E16,
                   ZP = z_piece<_Float16>();
     static_assert(ZP == E16, "16-byte z pieces");
     _Float16 ah[RG][VL], al[RG][VL], bh[NB][VL], bl[NB][VL];
@@ -651,13 +720,13 @@ __device__ inline void lr_rows_split(const MfEntry* __restrict__ ents, int e0, i
 // four lane groups of a row read one whole 128-byte line at once (an FP32 row
 // read 64 bytes at a time was fetched twice).  Temporal loads: a block's
 // lines are reused by the next step.
-template <int BL, class TD, int NB>
-__device__ inline void dense_rows(int leaf, const TD* __restrict__ Drm, const int32_t* __restrict__ nearPtr,
+template <int BL, int RG, class TD, int NB>
+__device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm, const int32_t* __restrict__ nearPtr,
                                   const MfNear* __restrict__ nearB, const TD* __restrict__ Xb, int lg, int lc,
-                                  int kvalid, typename Mfma<TD>::accv (&acc)[BL / 16][NB]) {
+                                  int kvalid, typename Mfma<TD>::accv (&acc)[RG][NB]) {
     using MD = Mfma<TD>;
     static_assert(MD::KL == 1, "dense blocks on the 16x16x4 shapes");
-    constexpr int NR = 16 * NB, EPL = 32 / sizeof(TD), SPB = BL / (4 * EPL), RG = BL / 16;
+    constexpr int NR = 16 * NB, EPL = 32 / sizeof(TD), SPB = BL / (4 * EPL);
     static_assert(SPB >= 1, "a step spans at most one block row");
     const int n0 = nearPtr ? nearPtr[leaf] : 0, n1 = nearPtr ? nearPtr[leaf + 1] : 0;
     const int total = (n1 - n0 + 1) * SPB;
@@ -668,7 +737,7 @@ __device__ inline void dense_rows(int leaf, const TD* __restrict__ Drm, const in
         const TD* Dq = q < n0 ? Drm + (size_t)leaf * BL * BL : (const TD*)nearB[q].d;
         const int cl = q < n0 ? leaf : nearB[q].colLeaf;
 #pragma unroll
-        for (int rg = 0; rg < RG; ++rg) vload(Dq + (16 * rg + lc) * BL + cc, A[rg]);
+        for (int rg = 0; rg < RG; ++rg) vload(Dq + (row0 + 16 * rg + lc) * BL + cc, A[rg]);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {  // right-hand sides past kvalid are zero in Xb: not loaded
             if (16 * nb + lc < kvalid) {
@@ -684,6 +753,23 @@ __device__ inline void dense_rows(int leaf, const TD* __restrict__ Drm, const in
             }
         }
     };
+    if constexpr (NB == 1) {
+        TD pa[kPipe][RG][EPL], pb[kPipe][NB][EPL];
+#pragma unroll
+        for (int d = 0; d < kPipe; ++d)
+            if (d < total) dload(d, pa[d], pb[d]);
+        for (int i0 = 0; i0 < total; i0 += kPipe)
+#pragma unroll
+            for (int d = 0; d < kPipe; ++d)
+                if (i0 + d < total) {
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e)
+#pragma unroll
+                        for (int rg = 0; rg < RG; ++rg) acc[rg][0] = MD::op(pa[d][rg][e], pb[d][0][e], acc[rg][0]);
+                    if (i0 + d + kPipe < total) dload(i0 + d + kPipe, pa[d], pb[d]);
+                }
+        return;
+    }
     dload(0, a, bx);
     for (int idx = 0; idx < total; ++idx) {
         const bool more = idx + 1 < total;
@@ -723,16 +809,16 @@ __device__ inline void dense_rows(int leaf, const TD* __restrict__ Drm, const in
 // operand is one 16-byte block of 8 right-hand-side rows.  Padding
 // positions hold the point (0, 0, 0): finite kernel values that meet zero
 // right-hand-side entries or land in discarded rows.
-template <int BL, int NB>
-__device__ inline void near_otf(int leaf, int w, const float4* __restrict__ PL, const double4* __restrict__ O,
+template <int BL, int RG, int NB>
+__device__ inline void near_otf(int leaf, int w, int row0, const float4* __restrict__ PL, const double4* __restrict__ O,
                                 float nlog2e, const int32_t* __restrict__ gnearPtr, const MfNear* __restrict__ gnear,
                                 const _Float16* __restrict__ Xh, const _Float16* __restrict__ Xl, int lg, int lc,
-                                int kvalid, v4f (&acc)[BL / 16][NB]) {
-    constexpr int RG = BL / 16, NR = 16 * NB, SH = 3;  // right-hand sides in blocks of 8 rows
+                                int kvalid, v4f (&acc)[RG][NB]) {
+    constexpr int NR = 16 * NB, SH = 3;  // right-hand sides in blocks of 8 rows
     float xl[RG][3];
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
-        const float4 p = PL[(size_t)leaf * BL + 16 * rg + lc];
+        const float4 p = PL[(size_t)leaf * BL + row0 + 16 * rg + lc];
         xl[rg][0] = p.x; xl[rg][1] = p.y; xl[rg][2] = p.z;
     }
     const double4 oi = O[leaf];
@@ -797,7 +883,8 @@ __device__ inline void near_otf(int leaf, int w, const float4* __restrict__ PL, 
 }
 
 // One workgroup of 4 waves per group of 4 consecutive leaves (S leaves in
-// all); wave w owns leaf 4g+w: its dense blocks and its entries (ptr, per
+// all; with RG < BL/16 row groups per wave, per 4 units of 16 RG rows); wave w
+// owns leaf 4g+w: its dense blocks and its entries (ptr, per
 // leaf), then -- grouped plans (64-row leaves) -- the tiles spanning the
 // whole group (gptr, per group; null otherwise).  The four waves walk the
 // shared list in the same order, so a tile's z block comes from HBM once per
@@ -811,7 +898,7 @@ __device__ inline void near_otf(int leaf, int w, const float4* __restrict__ PL, 
 // held as FP16 hi + lo (U, and z in right-hand-side units times 2^Ea) goes
 // first instead, its sum multiplied by hiMul = 2^(E - Ea) into the FP16
 // group's units.
-template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false>
+template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false, int RG = BL / 16>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 2 : 1))) k_mf_phase2g(int S, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
                                                     const int32_t* __restrict__ gptrA,
                                                     const MfEntry* __restrict__ gentA, const TA* __restrict__ ZA,
@@ -833,15 +920,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
     static_assert(sizeof(typename Mfma<TB>::acc_t) == sizeof(typename MA::acc_t) &&
                       sizeof(typename Mfma<TD>::acc_t) == sizeof(typename MA::acc_t),
                   "one accumulator type per launch");
-    constexpr int RG = BL / 16;
-    const int grp = xcd_local(blockIdx.x, gridDim.x);
+    constexpr int WPL = BL / 16 / RG;  // waves per leaf, RG 16-row groups each
+    const int blk = xcd_local(blockIdx.x, gridDim.x);
     // wave-uniform leaf (readfirstlane): scalar entry loads, no exec masks on
     // the entry loops.  FP64 phase 2 39.2 -> 38.1 ms at N = 2^20, 64
     // right-hand sides; the mixed kernel is slower that way (9.7 -> 10.2 ms,
     // measured) and keeps the per-lane index.
     const int w = sizeof(TA) == 8 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, lg = lane >> 4, lc = lane & 15;
-    const int leaf = 4 * grp + w;
+    const int unit = 4 * blk + w, leaf = unit / WPL, row0 = WPL > 1 ? 16 * RG * (unit % WPL) : 0;
+    const int grp = leaf >> 2, wl = leaf & 3;
     if (leaf >= S) return;  // last group of a plan whose leaf count is not a multiple of 4 (no barriers below)
     accv acc[RG][NB];
 #pragma unroll
@@ -849,24 +937,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[rg][nb] = accv{0, 0, 0, 0};
     if constexpr (SPA) {
-        lr_rows_split<BL, NB>(entA, ptrA[leaf], ptrA[leaf + 1], ZA, zLoA, uLoA, 0, lg, lc, kvalid, acc);
+        lr_rows_split<RG, NB>(entA, ptrA[leaf], ptrA[leaf + 1], ZA, zLoA, uLoA, row0, lg, lc, kvalid, acc);
         if (gptrA)
-            lr_rows_split<BL, NB>(gentA, gptrA[grp], gptrA[grp + 1], ZA, zLoA, uLoA, BL * w, lg, lc, kvalid, acc);
+            lr_rows_split<RG, NB>(gentA, gptrA[grp], gptrA[grp + 1], ZA, zLoA, uLoA, BL * wl + row0, lg, lc, kvalid, acc);
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) acc[rg][nb] *= hiMul;
     }
     if (ptrB) {
-        lr_rows<BL, false, TB, NB>(entB, ptrB[leaf], ptrB[leaf + 1], ZB, 0, lg, lc, kvalid, acc);
-        if (gptrB) lr_rows<BL, false, TB, NB>(gentB, gptrB[grp], gptrB[grp + 1], ZB, BL * w, lg, lc, kvalid, acc);
+        lr_rows<RG, false, TB, NB>(entB, ptrB[leaf], ptrB[leaf + 1], ZB, row0, lg, lc, kvalid, acc);
+        if (gptrB) lr_rows<RG, false, TB, NB>(gentB, gptrB[grp], gptrB[grp + 1], ZB, BL * wl + row0, lg, lc, kvalid, acc);
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) acc[rg][nb] *= (typename MA::acc_t)loMul;
     }
     if constexpr (std::is_same<TB, _Float16>::value && std::is_same<typename MA::accv, v4f>::value) {
-        if (P) near_otf<BL, NB>(leaf, w, P, O, nlog2e, nearPtr, nearB, Xh, Xl, lg, lc, kvalid, acc);
+        if (P) near_otf<BL, RG, NB>(leaf, wl, row0, P, O, nlog2e, nearPtr, nearB, Xh, Xl, lg, lc, kvalid, acc);
     }
     if (ptrB) {
 #pragma unroll
@@ -877,10 +965,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
             for (int rg = 0; rg < RG; ++rg) acc[rg][nb] *= f;
         }
     }
-    if (!P) dense_rows<BL, TD, NB>(leaf, Drm, nearPtr, nearB, Xb, lg, lc, kvalid, acc);
+    if (!P) dense_rows<BL, RG, TD, NB>(leaf, row0, Drm, nearPtr, nearB, Xb, lg, lc, kvalid, acc);
     if constexpr (!SPA) {
-        lr_rows<BL, UCM, TA, NB>(entA, ptrA[leaf], ptrA[leaf + 1], ZA, 0, lg, lc, kvalid, acc);
-        if (gptrA) lr_rows<BL, UCM, TA, NB>(gentA, gptrA[grp], gptrA[grp + 1], ZA, BL * w, lg, lc, kvalid, acc);
+        lr_rows<RG, UCM, TA, NB>(entA, ptrA[leaf], ptrA[leaf + 1], ZA, row0, lg, lc, kvalid, acc);
+        if (gptrA) lr_rows<RG, UCM, TA, NB>(gentA, gptrA[grp], gptrA[grp + 1], ZA, BL * wl + row0, lg, lc, kvalid, acc);
     }
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg)
@@ -889,7 +977,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
 #pragma unroll
             for (int v = 0; v < 4; ++v)
                 if (16 * nb + lc < kvalid)
-                    Y[(size_t)(16 * nb + lc) * ldy + (size_t)leaf * BL + 16 * rg + MA::out_row(lg, v)] = (TO)acc[rg][nb][v];
+                    Y[(size_t)(16 * nb + lc) * ldy + (size_t)leaf * BL + row0 + 16 * rg + MA::out_row(lg, v)] = (TO)acc[rg][nb][v];
 }
 
 // ---- right-hand-side conversion (mixed) ---------------------------------------
@@ -1809,12 +1897,25 @@ int phase1_chunk() {
     return v;
 }
 
+// Small plans give each wave less to do: phase 1 a wave per 16 columns of an
+// item instead of all 64, phase 2 a wave per 16 rows of a leaf instead of the
+// leaf.  A lone wave on a SIMD waits out every product (79 to 137 clocks per
+// FP64 16x16x4, nothing else to issue), so the chip's 1024 SIMDs need several
+// waves each; the same sums are formed in the same order either way.  16
+// right-hand sides, FP64 / mixed: N = 4096 2D 98 -> 58 / 66 -> 53 us, 16384 3D
+// 479 -> 244 / 237 -> 132; 64: 288 -> 171 / 98 -> 75, 1301 -> 730 / 351 ->
+// 228.  With enough waves the shared operands (right-hand sides, z) read more
+// often make it slower: N = 65536 2D (9200 items, 2048 leaves) phase 1 132 ->
+// 138, phase 2 141 -> 158 us; 60000 3D (1024 leaves of 64 rows) 648 -> 690.
+bool split_items(const MfGroup& G) { return G.numItems < 4096; }
+bool split_leaves(int S) { return S < 1024; }
+
 template <class T, int CG, int NB>
 void phase1(Context& c, MfGroup& G, const T* Xb, int sh, int kvalid, int xcdChunk = -1) {
     if (G.numItems == 0) return;
     const float* cs = G.colScaleV.n ? G.colScaleV.p : nullptr;
     const int chunk = xcdChunk >= 0 ? xcdChunk : phase1_chunk();
-    unsigned blocks = (unsigned)((G.numItems + 3) / 4);
+    unsigned blocks = (unsigned)(((int64_t)G.numItems * (kMfCols / 16 / CG) + 3) / 4);
     if (chunk > 0) blocks = (blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
     // FP64 groups read V in place (column-major) or from a fragment-ordered
     // copy: separate instantiations, so the in-place kernel's code is not
@@ -1839,9 +1940,11 @@ void phase1_split(Context& c, MfGroup& G, const _Float16* Xh, const _Float16* Xl
     HMX_CHECK(G.split == (sizeof(TZ) == 2 ? 2 : 1) && G.vfrag && G.colScaleV.n && Xl, HMX_ESTATE,
               "split phase 1: plan not built for it");
     const int chunk = phase1_chunk();
-    unsigned blocks = (unsigned)((G.numItems + 3) / 4);
+    const bool cols = split_items(G);
+    unsigned blocks = (unsigned)(((int64_t)G.numItems * (cols ? kMfCols / 16 : 1) + 3) / 4);
     if (chunk > 0) blocks = (blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
-    k_mf_phase1<_Float16, 4, NB, true, true, TZ><<<blocks, 256, 0, c.stream>>>(
+    auto k1 = cols ? k_mf_phase1<_Float16, 1, NB, true, true, TZ> : k_mf_phase1<_Float16, 4, NB, true, true, TZ>;
+    k1<<<blocks, 256, 0, c.stream>>>(
         G.items.p, G.numItems, chunk, Xh, sh, (float*)G.zpart.p, (TZ*)G.zt.p, G.zmap.p, G.colScaleV.p, kvalid, Xl,
         G.vLoOff, rhsScale, sizeof(TZ) == 2 ? split_zlo(G) : 0);
     HMX_LAUNCHED();
@@ -1876,7 +1979,8 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
     k_x_blocked<double, double><<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(
         tot, P.npad, NR, sh, X, ldx, kk, P.gather ? P.gmap.p : nullptr, nullptr, (double*)P.Xb.p);
     HMX_LAUNCHED();
-    phase1<double, 4, NB>(c, G, Xb, sh, kk, P.xcdChunk);  // 4 column groups = the 64 columns of an item
+    if (split_items(G)) phase1<double, 1, NB>(c, G, Xb, sh, kk, P.xcdChunk);
+    else phase1<double, 4, NB>(c, G, Xb, sh, kk, P.xcdChunk);  // 4 column groups = the 64 columns of an item
     ev.rec(c, 1);
     reduce_group<double, double>(c, G, NR);
     ev.rec(c, 2);
@@ -1885,11 +1989,18 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
     {
         const int* gp = G.grouped ? G.grpPtr.p : nullptr;
         const MfEntry* ge = G.grouped ? G.grpEntries.p : nullptr;
-        auto k2 = P.b == 64 ? (P.ucm ? k_mf_phase2g<64, true, double, double, double, NB, double>
-                                     : k_mf_phase2g<64, false, double, double, double, NB, double>)
-                            : (P.ucm ? k_mf_phase2g<32, true, double, double, double, NB, double>
-                                     : k_mf_phase2g<32, false, double, double, double, NB, double>);
-        k2<<<(P.S + 3) / 4, 256, 0, c.stream>>>(P.S, G.leafPtr.p, G.entries.p, gp, ge, (const double*)G.zt.p,
+        const bool split = split_leaves(P.S);
+        auto pick = [&](auto b, auto ucm) {
+            constexpr int B = decltype(b)::value;
+            constexpr bool U = decltype(ucm)::value;
+            return split ? k_mf_phase2g<B, U, double, double, double, NB, double, false, 1>
+                         : k_mf_phase2g<B, U, double, double, double, NB, double>;
+        };
+        using B64 = std::integral_constant<int, 64>;
+        using B32 = std::integral_constant<int, 32>;
+        auto k2 = P.b == 64 ? (P.ucm ? pick(B64{}, std::true_type{}) : pick(B64{}, std::false_type{}))
+                            : (P.ucm ? pick(B32{}, std::true_type{}) : pick(B32{}, std::false_type{}));
+        k2<<<(P.S * (split ? P.b / 16 : 1) + 3) / 4, 256, 0, c.stream>>>(P.S, G.leafPtr.p, G.entries.p, gp, ge, (const double*)G.zt.p,
                                                 nullptr, nullptr, nullptr, nullptr, nullptr, (const double*)P.Drm.p,
                                                 P.nearPtr.p, P.near.p, Xb, Yo, ldo, kk, nullptr, 1.f, nullptr, nullptr,
                                                 0.f, nullptr, nullptr, 0, 0, 1.f);
@@ -1927,7 +2038,8 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
     if (Ghi.split == 2) phase1_split<NB, _Float16>(c, Ghi, P.X16.p, P.X16lo.p, sh16, kk, nullptr);
     else if (Ghi.split == 1) phase1_split<NB, float>(c, Ghi, P.X16.p, P.X16lo.p, sh16, kk, P.xscale.p);
     else phase1<float, 4, NB>(c, Ghi, Xb, sh32, kk);
-    phase1<_Float16, 4, NB>(c, Glo, P.X16.p, sh16, kk);
+    if (split_items(Glo)) phase1<_Float16, 1, NB>(c, Glo, P.X16.p, sh16, kk);
+    else phase1<_Float16, 4, NB>(c, Glo, P.X16.p, sh16, kk);
     ev.rec(c, 1);
     if (Ghi.split == 2) reduce_group<float, _Float16>(c, Ghi, NR, nullptr, split_zlo(Ghi));
     else reduce_group<float, float>(c, Ghi, NR, Ghi.split ? P.xscale.p : nullptr);
@@ -1939,8 +2051,9 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
         const bool gr = Ghi.grouped && Glo.grouped;
         const bool spa = Ghi.split == 2;
         // a split group's z is FP16 hi + lo (the kernel's ZA), else FP32
+        const bool split = !spa && split_leaves(P.S);
         auto launch = [&](auto k2, const auto* za) {
-            k2<<<(P.S + 3) / 4, 256, 0, c.stream>>>(
+            k2<<<(P.S * (split ? P.b / 16 : 1) + 3) / 4, 256, 0, c.stream>>>(
                 P.S, Ghi.leafPtr.p, Ghi.entries.p, gr ? Ghi.grpPtr.p : nullptr, gr ? Ghi.grpEntries.p : nullptr, za,
                 Glo.leafPtr.p, Glo.entries.p, gr ? Glo.grpPtr.p : nullptr, gr ? Glo.grpEntries.p : nullptr,
                 (const _Float16*)Glo.zt.p, (const float*)P.Drm.p, P.nearOtf ? P.gnearPtr.p : P.nearPtr.p,
@@ -1953,6 +2066,8 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
         const float* zf = (const float*)Ghi.zt.p;
         if (spa && P.b == 64) launch(k_mf_phase2g<64, false, float, _Float16, _Float16, NB, float, true>, zh);
         else if (spa) launch(k_mf_phase2g<32, false, float, _Float16, _Float16, NB, float, true>, zh);
+        else if (split && P.b == 64) launch(k_mf_phase2g<64, false, float, float, _Float16, NB, float, false, 1>, zf);
+        else if (split) launch(k_mf_phase2g<32, false, float, float, _Float16, NB, float, false, 1>, zf);
         else if (P.b == 64) launch(k_mf_phase2g<64, false, float, float, _Float16, NB, float>, zf);
         else launch(k_mf_phase2g<32, false, float, float, _Float16, NB, float>, zf);
     }

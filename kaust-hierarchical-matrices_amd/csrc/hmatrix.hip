@@ -361,28 +361,14 @@ __global__ void __launch_bounds__(256) k_dir_sum(LrLevel L, int splits, const do
     Yout[(size_t)p * bstride + (size_t)t * per + e] = v;
 }
 
-// 4 consecutive doubles of a column (32-byte aligned: columns start at
-// multiples of 64 rows, lanes at multiples of 4)
-__device__ inline void ld4(const double* p, bool ok, double (&o)[4]) {
-    const double2 z = make_double2(0.0, 0.0);
-    const double2 a = ok ? reinterpret_cast<const double2*>(p)[0] : z;
-    const double2 b = ok ? reinterpret_cast<const double2*>(p)[1] : z;
-    o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
-}
-
 // W[t][s*k + a] = sum_i Q_t[a*m+i] B_t[s*m+i], a < k_t, on the FP64 matrix
-// cores: one workgroup per 16 basis columns of a tile, its waves deal out the
-// rows, and their partial 16 x 16 blocks are added in wave order.
-// A lane takes 4 consecutive rows of one column (16 columns x 128 contiguous
-// bytes per load pair), two 16-row steps in flight: the same rows one double
-// a lane at a time ran one dependent load per product.  16 waves from 1024
-// rows on, where the few tiles of a level leave CUs free and the run of rows
-// per wave is what bounds it.  N = 65536 3D build, all levels: 7.2 ms, 8.7
-// before.
+// cores: one workgroup per 16 basis columns of a tile, its four waves take
+// a quarter of the rows each (lane l holds Q^T[a0 + l%16][i + l/16] and
+// B[i + l/16][l%16] for the step at row i), and the four partial 16 x 16
+// blocks are added in wave order.
 // mode 0: B = Y (16 columns, tile still iterating); mode 2: B = accepted block (na columns)
-template <int NW>
-__global__ void __launch_bounds__(64 * NW) k_lr_dot(LrLevel L, int mode) {
-    __shared__ double red[NW][64][4];
+__global__ void __launch_bounds__(256) k_lr_dot(LrLevel L, int mode) {
+    __shared__ double red[3][64][4];
     const int t = blockIdx.y;
     const LrState& S = L.st[t];
     // before the decision step the tile must still be iterating; after it,
@@ -395,31 +381,24 @@ __global__ void __launch_bounds__(64 * NW) k_lr_dot(LrLevel L, int mode) {
     const int m = L.m;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
     const bool av = a0 + lc < K, sv = lc < C;
-    const double* qa = L.Q + (size_t)t * m * L.capQ + (size_t)(av ? a0 + lc : 0) * m + 4 * lg;
-    const double* bs = (mode == 0 ? L.Y : L.Ya) + (size_t)t * m * kB16 + (size_t)(sv ? lc : 0) * m + 4 * lg;
-    // chunks of 16 rows (128 bytes a column) dealt to the waves in turn: the
-    // columns lie a power of two apart, so waves far apart in a column would
-    // all read from one memory channel
+    const double* qa = L.Q + (size_t)t * m * L.capQ + (size_t)(av ? a0 + lc : 0) * m;
+    const double* bs = (mode == 0 ? L.Y : L.Ya) + (size_t)t * m * kB16 + (size_t)(sv ? lc : 0) * m;
+    const int part = m / 4, i0 = w * part;  // m is a multiple of 64
     v4d_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-    for (int i = 16 * w; i < m; i += 16 * NW) {
-        double x[4], y[4];
-        ld4(qa + i, av, x);
-        ld4(bs + i, sv, y);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e], y[e], acc, 0, 0, 0);
+    for (int i = i0; i < i0 + part; i += 4) {
+        const double x = av ? qa[i + lg] : 0.0;
+        const double y = sv ? bs[i + lg] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc, 0, 0, 0);
     }
     if (w > 0)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) red[w][lane][v] = acc[v];
+        for (int v = 0; v < 4; ++v) red[w - 1][lane][v] = acc[v];
     __syncthreads();
     if (w > 0) return;
     double* out = L.W + (size_t)t * L.capQ * kB16;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        double r = acc[v];
-#pragma unroll
-        for (int q = 1; q < NW; ++q) r += red[q][lane][v];
+        const double r = ((acc[v] + red[0][lane][v]) + red[1][lane][v]) + red[2][lane][v];
         const int a = a0 + 4 * v + lg;  // output row 4v + l/16, column l%16
         if (a < K && lc < C) out[lc * K + a] = r;
     }
@@ -446,21 +425,31 @@ __global__ void __launch_bounds__(256) k_lr_update(LrLevel L, int mode) {
     v4d_t acc;
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[v] = sv ? Y[(size_t)lc * m + row0 + 4 * v + lg] : 0.0;
-    for (int a = 0; a < k; a += 16) {  // the loads of 4 steps together
-        double x[4], y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int q = a + 4 * e + lg;
-            const bool ok = q < k;
-            x[e] = ok ? Q[(size_t)q * m + row0 + lc] : 0.0;
-            y[e] = ok && sv ? -W[(size_t)lc * k + q] : 0.0;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e], y[e], acc, 0, 0, 0);
+    for (int a = 0; a < k; a += 4) {
+        const bool ok = a + lg < k;
+        const double x = ok ? Q[(size_t)(a + lg) * m + row0 + lc] : 0.0;
+        const double y = ok && sv ? -W[(size_t)lc * k + a + lg] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc, 0, 0, 0);
     }
     if (sv)
 #pragma unroll
         for (int v = 0; v < 4; ++v) Y[(size_t)lc * m + row0 + 4 * v + lg] = acc[v];
+}
+
+// sum over the block; every thread receives the identical value.  red holds
+// two slots of 16: consecutive calls alternate (parity), so one barrier per
+// call suffices -- a thread reaches the call after next only once every
+// thread has passed the next call's barrier, i.e. has read this one's slot.
+__device__ inline double block_sum(double v, double* red, int& parity) {
+    v = wave_sum_dpp(v);
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double* slot = red + 16 * parity;
+    parity ^= 1;
+    if ((threadIdx.x & 63) == 0) slot[w] = v;
+    __syncthreads();
+    double s = 0.0;
+    for (int q = 0; q < nw; ++q) s += slot[q];
+    return s;
 }
 
 // One wave per tile for tiles of m <= 512 rows (R = m / 64 rows per lane):
@@ -521,6 +510,107 @@ __global__ void __launch_bounds__(64) k_lr_decide_w(LrLevel L) {
     if (lane == 0) { S.na = na; S.small_run = small; S.converged = conv; S.capped = capped; }
 }
 
+// The same decisions for tiles of 1024 and 2048 rows: four waves, thread
+// t owning rows t + 256 i (i < R = m / 256), the current column and the
+// block's accepted columns in registers, one barrier per sum (block_sum)
+template <int R>
+__global__ void __launch_bounds__(256) k_lr_decide_b(LrLevel L) {
+    __shared__ double red[32];
+    int parity = 0;
+    const int t = blockIdx.x, tid = threadIdx.x;
+    LrState& S = L.st[t];
+    if (!lr_active(S, L.tp[t].maxRank)) {
+        if (tid == 0) S.na = 0;
+        return;
+    }
+    const int m = L.m;
+    const double* Y = L.Y + (size_t)t * m * kB16;
+    double* Qb = L.Ya + (size_t)t * m * kB16;
+    double qb[kB16][R];
+    int na = 0, small = S.small_run, conv = 0, capped = 0;
+    const int capleft = L.tp[t].maxRank - S.k;
+    const double tau = L.tp[t].tau;
+    for (int j = 0; j < kB16; ++j) {
+        double y[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) y[r] = Y[(size_t)j * m + tid + 256 * r];
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass)
+#pragma unroll
+            for (int a = 0; a < kB16; ++a)
+                if (a < na) {
+                    double p = 0.0;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) p += qb[a][r] * y[r];
+                    const double d = block_sum(p, red, parity);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) y[r] -= qb[a][r] * d;
+                }
+        double p = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) p += y[r] * y[r];
+        const double nu = sqrt(block_sum(p, red, parity));
+        if (nu > tau) {
+            if (na >= capleft) { capped = 1; break; }
+#pragma unroll
+            for (int a = 0; a < kB16; ++a)
+                if (a == na)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) qb[a][r] = y[r] / nu;
+#pragma unroll
+            for (int r = 0; r < R; ++r) Qb[(size_t)na * m + tid + 256 * r] = y[r] / nu;
+            ++na;
+            small = 0;
+        } else if (++small >= L.r) {
+            conv = 1;
+            break;
+        }
+    }
+    if (tid == 0) { S.na = na; S.small_run = small; S.converged = conv; S.capped = capped; }
+}
+
+// k_lr_renorm for tiles of 1024 and 2048 rows: four waves, registers
+template <int R>
+__global__ void __launch_bounds__(256) k_lr_renorm_b(LrLevel L) {
+    __shared__ double red[32];
+    int parity = 0;
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const LrState& S = L.st[t];
+    const int na = S.na;
+    if (na == 0) return;
+    const int m = L.m;
+    double* Qb = L.Ya + (size_t)t * m * kB16;
+    double* Q = L.Q + (size_t)t * m * L.capQ;
+    double qb[kB16][R];
+#pragma unroll
+    for (int j = 0; j < kB16; ++j)
+        if (j < na) {
+            double q[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) q[r] = Qb[(size_t)j * m + tid + 256 * r];
+#pragma unroll
+            for (int a = 0; a < j; ++a) {
+                double p = 0.0;
+#pragma unroll
+                for (int r = 0; r < R; ++r) p += qb[a][r] * q[r];
+                const double d = block_sum(p, red, parity);
+#pragma unroll
+                for (int r = 0; r < R; ++r) q[r] -= qb[a][r] * d;
+            }
+            double p = 0.0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) p += q[r] * q[r];
+            const double nu = sqrt(block_sum(p, red, parity));
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const double v = q[r] / nu;
+                qb[j][r] = v;
+                Qb[(size_t)j * m + tid + 256 * r] = v;
+                Q[(size_t)(S.k + j) * m + tid + 256 * r] = v;
+            }
+        }
+}
+
 // k_lr_renorm for tiles of m <= 512 rows, one wave per tile, registers only
 template <int R>
 __global__ void __launch_bounds__(64) k_lr_renorm_w(LrLevel L) {
@@ -561,207 +651,80 @@ __global__ void __launch_bounds__(64) k_lr_renorm_w(LrLevel L) {
         }
 }
 
-// out[a][c] = sum over rows of A's column a and B's column c (a lane's column
-// is l % 16; columns not ok count as zero), m rows in chunks of 16 dealt to
-// the workgroup's 16 waves, whose partial blocks are added in wave order.
-// out is complete after the closing barrier.
-__device__ inline void tall_products(const double* A, bool aok, const double* B, bool bok,
-                                     int m, double (*red)[64][4], double (*out)[17]) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
-    const double* a = A + (size_t)(aok ? lc : 0) * m + 4 * lg;
-    const double* b = B + (size_t)(bok ? lc : 0) * m + 4 * lg;
-    v4d_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-    for (int i = 16 * w; i < m; i += 256) {
-        double x[4], y[4];
-        ld4(a + i, aok, x);
-        ld4(b + i, bok, y);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e], y[e], acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) red[w][lane][v] = acc[v];
-    __syncthreads();
-    if (w < 4) {  // wave w folds register w: row 4w + l/16, column l%16
-        double r = red[0][lane][w];
-#pragma unroll
-        for (int q = 1; q < 16; ++q) r += red[q][lane][w];
-        out[4 * w + lg][lc] = r;
-    }
-    __syncthreads();
-}
-
-// Columns c < 16 of dst, where ok: dst_c = init_c + sum_k coef[k] src_k with
-// lane (lg, lc) holding coef(k = 4e + lg, c = lc) in a[e]; src columns not in
-// [k0, k1) count as zero.  A lane reads row lc of columns 4e + lg and stores
-// row lc of columns 4v + lg: 128 contiguous bytes per column.
-template <bool INIT>
-__device__ inline void tall_combine(const double (&a)[4], const double* src, int k0, int k1, double* dst, int c0,
-                                    int c1, int m) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
-    for (int i = 16 * w; i < m; i += 256) {
-        double x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = 4 * e + lg;
-            x[e] = k >= k0 && k < k1 ? src[(size_t)k * m + i + lc] : 0.0;
-        }
-        v4d_t o = {0.0, 0.0, 0.0, 0.0};
-        if (INIT)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int c = 4 * v + lg;
-                o[v] = c >= c0 && c < c1 ? dst[(size_t)c * m + i + lc] : 0.0;
-            }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], x[e], o, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int c = 4 * v + lg;
-            if (c >= c0 && c < c1) dst[(size_t)c * m + i + lc] = o[v];
-        }
-    }
-}
-
-// Tiles of 1024 rows and more (and the short ones below 64), one workgroup
-// of 16 waves per tile: the block's columns in order, a column accepted when
-// its norm after orthogonalisation against the block's accepted columns
-// exceeds tau, the tile converged after r small ones in a row.
-//
-// The norms come from the Gram matrix of the columns: elimination in column
-// order leaves the squared norm of a column's orthogonal part on the
-// diagonal, to rounding relative to the column's own squared norm.  That
-// decides a column as long as its part is not below 1e-3 of the column (the
-// decided norms are then exact to 1e-10), or is below tau for certain; the
-// first column of which neither holds ends the panel: the accepted columns
-// so far are formed (Y times the triangular factor's inverse), the columns
-// left are projected against them explicitly, twice, and their own Gram
-// matrix goes on from there.  Sequential Gram-Schmidt makes a round of
-// workgroup sums per pair of columns and sweep; this makes one pass of
-// products and one of updates over the block per panel, on the matrix cores,
-// and one or two panels are usual.  (k_lr_renorm orthonormalises the block
-// to rounding afterwards.)
-//
-// Bound by one CU's reads of the block (128 m bytes a pass).  N = 65536 3D
-// build, the levels of 1024 to 8192 rows: 2.8 ms; a round of sums per
-// coefficient took 15.1, two rounds per column 10.0.
+// One workgroup per tile: column-by-column decisions on explicitly projected
+// vectors (two modified Gram-Schmidt sweeps against the block's accepted
+// columns, accept when the norm exceeds tau).  Threads own fixed rows, so
+// only the reductions need the workgroup barrier.
 __global__ void __launch_bounds__(1024) k_lr_decide(LrLevel L) {
-    __shared__ double red[16][64][4], G[16][17], T[16][17], g0[16];
-    __shared__ int idx[16];
-    const int t = blockIdx.x, tid = threadIdx.x;
+    __shared__ double red[32];
+    int parity = 0;
+    const int t = blockIdx.x;
     LrState& S = L.st[t];
     if (!lr_active(S, L.tp[t].maxRank)) {
-        if (tid == 0) S.na = 0;
+        if (threadIdx.x == 0) S.na = 0;
         return;
     }
-    const int lane = tid & 63, lc = lane & 15, lg = lane >> 4;
-    const int m = L.m;
+    const int m = L.m, nthr = blockDim.x, tid = threadIdx.x;
     double* Y = L.Y + (size_t)t * m * kB16;
     double* Qb = L.Ya + (size_t)t * m * kB16;
     int na = 0, small = S.small_run, conv = 0, capped = 0;
     const int capleft = L.tp[t].maxRank - S.k;
     const double tau = L.tp[t].tau;
-    for (int j0 = 0; j0 < kB16;) {
-        tall_products(Y, lc >= j0, Y, lc >= j0, m, red, G);
-        const int q = tid >> 4;  // thread (row q, column lc) of G and T
-        const bool el = tid < 256;
-        if (el) T[q][lc] = q == lc ? 1.0 : 0.0;
-        if (tid < 16) g0[tid] = G[tid][tid];
-        __syncthreads();
-        int cnt = 0, j = j0;
-        for (; j < kB16; ++j) {  // the same in every thread
-            const double d = G[j][j];
-            bool accept = false;
-            if (j == j0 || d > 1e-6 * g0[j]) accept = sqrt(d) > tau;
-            else if (!(sqrt((d > 0.0 ? d : 0.0) + 1e-12 * g0[j]) < 0.99 * tau)) break;  // needs the explicit projection
-            if (!accept) {
-                if (++small >= L.r) { conv = 1; break; }
-                continue;
+    for (int j = 0; j < kB16; ++j) {
+        double* y = Y + (size_t)j * m;
+        for (int pass = 0; pass < 2; ++pass)
+            for (int a = 0; a < na; ++a) {
+                const double* qa = Qb + (size_t)a * m;
+                double p = 0.0;
+                for (int i = tid; i < m; i += nthr) p += qa[i] * y[i];
+                const double d = block_sum(p, red, parity);
+                for (int i = tid; i < m; i += nthr) y[i] -= qa[i] * d;
             }
-            if (na + cnt >= capleft) { capped = 1; break; }
+        double p = 0.0;
+        for (int i = tid; i < m; i += nthr) p += y[i] * y[i];
+        const double nu = sqrt(block_sum(p, red, parity));
+        if (nu > tau) {
+            if (na >= capleft) { capped = 1; break; }
+            for (int i = tid; i < m; i += nthr) Qb[(size_t)na * m + i] = y[i] / nu;
+            ++na;
             small = 0;
-            if (tid == 0) idx[cnt] = j;
-            ++cnt;
-            if (el && q > j) {
-                const double f = G[j][q] / d;
-                const double g = G[q][lc] - f * G[j][lc], e = T[q][lc] - f * T[j][lc];
-                G[q][lc] = g;
-                T[q][lc] = e;
-            }
-            __syncthreads();
+        } else if (++small >= L.r) {
+            conv = 1;
+            break;
         }
-        __syncthreads();
-        const bool done = conv || capped || j == kB16;
-        if (cnt > 0) {
-            double a[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                a[e] = lc < cnt ? T[idx[lc]][4 * e + lg] / sqrt(G[idx[lc]][idx[lc]]) : 0.0;
-            tall_combine<false>(a, Y, j0, j, Qb + (size_t)na * m, 0, cnt, m);
-            na += cnt;
-        }
-        if (done) break;
-        for (int rep = 0; rep < 2; ++rep) {
-            __syncthreads();
-            tall_products(Qb, lc < na, Y, lc >= j, m, red, G);
-            double a[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[e] = 4 * e + lg < na && lc >= j ? -G[4 * e + lg][lc] : 0.0;
-            tall_combine<true>(a, Qb, 0, na, Y, j, kB16, m);
-        }
-        __syncthreads();
-        j0 = j;
     }
     if (tid == 0) { S.na = na; S.small_run = small; S.converged = conv; S.capped = capped; }
 }
 
-// Tiles of 1024 rows and more (and below 64), after the accepted columns were projected
-// against Q: orthonormalise the block and append it to Q.  The columns are
-// orthonormal up to what the projection took off (rounding relative to the
-// sampled block), so their Gram matrix G is close to 1 and one Cholesky
-// factorisation G = R^T R gives what a modified Gram-Schmidt sweep would, to
-// rounding: B R^-1, one pass of products and one of updates on the matrix
-// cores instead of a round of sums per pair of columns.  A block that is not
-// close (tolerances near rounding) takes the step again, at most twice more.
-// N = 65536 3D build, levels of 1024 to 8192 rows: 1.9 ms, 7.4 before.
+// After the accepted columns were projected against Q: one more modified
+// Gram-Schmidt sweep inside the block, normalise, append to Q.
 __global__ void __launch_bounds__(1024) k_lr_renorm(LrLevel L) {
-    __shared__ double red[16][64][4], G[16][17], T[16][17];
+    __shared__ double red[32];
+    int parity = 0;
     const int t = blockIdx.x;
     const LrState& S = L.st[t];
     const int na = S.na;
     if (na == 0) return;
-    const int m = L.m;
-    const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+    const int m = L.m, nthr = blockDim.x, tid = threadIdx.x;
     double* Qb = L.Ya + (size_t)t * m * kB16;
-    double* Q = L.Q + (size_t)t * m * L.capQ + (size_t)S.k * m;
-    for (int pass = 0; pass < 3; ++pass) {
-        tall_products(Qb, lc < na, Qb, lc < na, m, red, G);
-        // G = R^T R by elimination, thread (row q, column lc); the same row
-        // operations on the identity give R^-1 = (rows of T / pivots' roots)^T
-        const int q = threadIdx.x >> 4;
-        const bool el = threadIdx.x < 256;
-        bool far = false;
-        if (el) {
-            T[q][lc] = q == lc ? 1.0 : 0.0;
-            far = q < na && lc < na && !(fabs(G[q][lc] - (q == lc ? 1.0 : 0.0)) <= 1e-3);
+    double* Q = L.Q + (size_t)t * m * L.capQ;
+    for (int j = 0; j < na; ++j) {
+        double* q = Qb + (size_t)j * m;
+        for (int a = 0; a < j; ++a) {
+            const double* qa = Qb + (size_t)a * m;
+            double p = 0.0;
+            for (int i = tid; i < m; i += nthr) p += qa[i] * q[i];
+            const double d = block_sum(p, red, parity);
+            for (int i = tid; i < m; i += nthr) q[i] -= qa[i] * d;
         }
-        const bool more = __syncthreads_or(far) && pass < 2;
-        for (int a = 0; a < na; ++a) {
-            if (el && q > a && q < na) {
-                const double f = G[a][q] / G[a][a];
-                const double g = G[q][lc] - f * G[a][lc], e = T[q][lc] - f * T[a][lc];
-                G[q][lc] = g;
-                T[q][lc] = e;
-            }
-            __syncthreads();
+        double p = 0.0;
+        for (int i = tid; i < m; i += nthr) p += q[i] * q[i];
+        const double nu = sqrt(block_sum(p, red, parity));
+        for (int i = tid; i < m; i += nthr) {
+            const double v = q[i] / nu;
+            q[i] = v;
+            Q[(size_t)(S.k + j) * m + i] = v;
         }
-        double a[4];  // column lc of R^-1
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            a[e] = lc < na && 4 * e + lg < na ? T[lc][4 * e + lg] / sqrt(G[lc][lc]) : 0.0;
-        tall_combine<false>(a, Qb, 0, na, more ? Qb : Q, 0, na, m);
-        if (!more) break;
-        __syncthreads();
     }
 }
 
@@ -1136,12 +1099,7 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
     HMX_LAUNCHED();
     const auto tB = std::chrono::steady_clock::now();
     const unsigned rowBlocks = (unsigned)((m + 63) / 64);
-    auto dot = [&](unsigned kb, int mode) {
-        if (m >= 1024) k_lr_dot<16><<<dim3(kb, T), 1024, 0, c.stream>>>(L, mode);
-        else if (m >= 64) k_lr_dot<4><<<dim3(kb, T), 256, 0, c.stream>>>(L, mode);
-        else k_lr_dot<1><<<dim3(kb, T), 64, 0, c.stream>>>(L, mode);
-        HMX_LAUNCHED();
-    };
+    const unsigned wgThreads = m >= 4096 ? 1024u : 256u;
     int kmax = 0, preStart = 0, preN = 0, sweeps = 0;
     int active = T;  // tiles still iterating (the count k_lr_commit reports)
     const int maxIters = (2 * maxRank + araR) / kB16 + 2;
@@ -1187,7 +1145,8 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         }
         const unsigned kb = (unsigned)std::max(1, (kmax + 15) / 16);
         for (int pass = 0; pass < 2 && kmax > 0; ++pass) {
-            dot(kb, 0);
+            k_lr_dot<<<dim3(kb, T), 256, 0, c.stream>>>(L, 0);
+            HMX_LAUNCHED();
             k_lr_update<<<dim3(rowBlocks, T), 256, 0, c.stream>>>(L, 0);
             HMX_LAUNCHED();
         }
@@ -1195,10 +1154,13 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         else if (m == 128) k_lr_decide_w<2><<<T, 64, 0, c.stream>>>(L);
         else if (m == 256) k_lr_decide_w<4><<<T, 64, 0, c.stream>>>(L);
         else if (m == 512) k_lr_decide_w<8><<<T, 64, 0, c.stream>>>(L);
-        else k_lr_decide<<<T, 1024, 0, c.stream>>>(L);
+        else if (m == 1024) k_lr_decide_b<4><<<T, 256, 0, c.stream>>>(L);
+        else if (m == 2048) k_lr_decide_b<8><<<T, 256, 0, c.stream>>>(L);
+        else k_lr_decide<<<T, wgThreads, 0, c.stream>>>(L);
         HMX_LAUNCHED();
         if (kmax > 0) {
-            dot(kb, 2);
+            k_lr_dot<<<dim3(kb, T), 256, 0, c.stream>>>(L, 2);
+            HMX_LAUNCHED();
             k_lr_update<<<dim3(rowBlocks, T), 256, 0, c.stream>>>(L, 2);
             HMX_LAUNCHED();
         }
@@ -1206,7 +1168,9 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         else if (m == 128) k_lr_renorm_w<2><<<T, 64, 0, c.stream>>>(L);
         else if (m == 256) k_lr_renorm_w<4><<<T, 64, 0, c.stream>>>(L);
         else if (m == 512) k_lr_renorm_w<8><<<T, 64, 0, c.stream>>>(L);
-        else k_lr_renorm<<<T, 1024, 0, c.stream>>>(L);
+        else if (m == 1024) k_lr_renorm_b<4><<<T, 256, 0, c.stream>>>(L);
+        else if (m == 2048) k_lr_renorm_b<8><<<T, 256, 0, c.stream>>>(L);
+        else k_lr_renorm<<<T, wgThreads, 0, c.stream>>>(L);
         HMX_LAUNCHED();
         HMX_HIP(hipMemsetAsync(ws.flags.p, 0, 2 * sizeof(int), c.stream));
         k_lr_commit<<<(T + 255) / 256, 256, 0, c.stream>>>(L, ws.flags.p);

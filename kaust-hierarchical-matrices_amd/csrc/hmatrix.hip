@@ -24,6 +24,7 @@ namespace hmx {
 double ara_threshold(double tol);
 
 constexpr int kB16 = 16;
+typedef double v4d_t __attribute__((ext_vector_type(4)));
 
 struct LrState {
     int k, small_run, converged, capped, na;
@@ -81,56 +82,109 @@ __global__ void __launch_bounds__(256) k_lr_omega(LrLevel L, int it, int nb, int
     L.Om[(size_t)t * L.m * wd + e] = gauss_at(L.seed, kTagOmega, L.tp[t].opid, (uint32_t)(it * kB16 + j), (uint32_t)c);
 }
 
-// Y rows of row-leaf i of tile t: sum over column leaves j of U_ij (V_ij^T Om_j)
-template <int BMAX>
-__global__ void __launch_bounds__(256) k_lr_sample(LrLevel L) {
-    __shared__ double sV[BMAX * BMAX], sU[BMAX * BMAX], sO[BMAX * kB16], sT[BMAX * kB16];
-    const int t = blockIdx.y, i = blockIdx.x, b = L.b, m = L.m;
-    if (!lr_active(L.st[t], L.tp[t].maxRank)) return;
-    const double* Om = L.Om + (size_t)t * m * kB16;
-    double acc[(BMAX * kB16 + 255) / 256];
+// TLR-sum sampler: one leaf's rows of A X or A^T X for a tile A that is the sum
+// of its leaf tiles' factors, sum over the other side's leaves of
+// F_out (F_in^T X_leaf).
+//   TRANSPOSED = false: row leaf o of Y = A Om (F_out = U, F_in = V, 16 columns)
+//   TRANSPOSED = true: column leaf o of B = A^T Q (F_out = V, F_in = U), the
+//   basis columns 64 blockIdx.x ... of every tile
+// RG = 16-row groups of a leaf (rows past b masked), CB = 16-column blocks.
+//
+// The workgroup's waves take the leaves in turn, each on its own: the first
+// product's result registers (lane (lg, lc), register v: factor column 4v +
+// lg, X column lc) are the second's operand as they stand, so nothing goes
+// through LDS and no wave waits for another until the waves' sums are folded
+// in order at the end.  Bound by the latency of a leaf's loads (rank, then
+// factors: 128-byte lines) for the few tiles of the top levels, by the
+XX
+// A^T Q together; a workgroup per leaf with factors and products staged in
+// LDS, three barriers per leaf, took 7.5.
+template <int RG, int CB, bool TRANSPOSED>
+__global__ void __launch_bounds__(256) k_lr_leaf_sum(LrLevel L, double* __restrict__ Bout) {
+    __shared__ double red[3][RG * CB * 4][64];
+    const int t = blockIdx.z, o = blockIdx.y, c0 = blockIdx.x * 16 * CB, b = L.b, m = L.m;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, lg = lane >> 4, lc = lane & 15;
+    int cols;
+    if (TRANSPOSED) {
+        cols = L.st[t].k - c0;
+        if (cols <= 0) return;
+    } else {
+        if (!lr_active(L.st[t], L.tp[t].maxRank)) return;
+        cols = kB16;
+    }
+    const double* X = TRANSPOSED ? L.Q + (size_t)t * m * L.capQ + (size_t)c0 * m : L.Om + (size_t)t * m * kB16;
+    v4d_t acc[RG][CB];
 #pragma unroll
-    for (int q = 0; q < (BMAX * kB16 + 255) / 256; ++q) acc[q] = 0.0;
-    for (int j = 0; j < L.bus; ++j) {
-        int64_t mo = L.first[t] + (int64_t)morton_xy((uint32_t)j, (uint32_t)i);
-        int rk = L.ranksMO[mo];
+    for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) acc[rg][cb] = v4d_t{0.0, 0.0, 0.0, 0.0};
+    for (int q = w; q < L.bus; q += nw) {
+        const int64_t mo = L.first[t] + (int64_t)(TRANSPOSED ? morton_xy((uint32_t)o, (uint32_t)q)
+                                                             : morton_xy((uint32_t)q, (uint32_t)o));
+        const int rk = L.ranksMO[mo];
         if (rk == 0) continue;
-        const double* U = L.UMO + (size_t)L.offMO[mo] * b;
-        const double* V = L.VMO + (size_t)L.offMO[mo] * b;
-        for (int e = threadIdx.x; e < rk * b; e += 256) { sU[e] = U[e]; sV[e] = V[e]; }
-        for (int e = threadIdx.x; e < b * kB16; e += 256) {
-            int s = e / b, x = e % b;
-            sO[e] = Om[(size_t)s * m + (size_t)j * b + x];
-        }
-        __syncthreads();
-        for (int e = threadIdx.x; e < rk * kB16; e += 256) {  // sT[s*rk + a] = V_a . Om_s
-            int s = e / rk, a = e % rk;
-            double v = 0.0;
-            for (int x = 0; x < b; ++x) v += sV[a * b + x] * sO[s * b + x];
-            sT[e] = v;
-        }
-        __syncthreads();
+        const double* Fin = (TRANSPOSED ? L.UMO : L.VMO) + (size_t)L.offMO[mo] * b;
+        const double* Fout = (TRANSPOSED ? L.VMO : L.UMO) + (size_t)L.offMO[mo] * b;
+        const double* Xq = X + (size_t)q * b;
+        for (int a0 = 0; a0 < rk; a0 += 16) {
+            v4d_t tt[CB];
 #pragma unroll
-        for (int q = 0; q < (BMAX * kB16 + 255) / 256; ++q) {
-            int e = threadIdx.x + q * 256;
-            if (e < b * kB16) {
-                int s = e / b, x = e % b;
-                double v = acc[q];
-                for (int a = 0; a < rk; ++a) v += sU[a * b + x] * sT[s * rk + a];
-                acc[q] = v;
+            for (int cb = 0; cb < CB; ++cb) tt[cb] = v4d_t{0.0, 0.0, 0.0, 0.0};
+            double fo[4][RG];
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int rg = 0; rg < RG; ++rg)
+                    fo[v][rg] = a0 + 4 * v + lg < rk && 16 * rg + lc < b
+                                    ? Fout[(size_t)(a0 + 4 * v + lg) * b + 16 * rg + lc] : 0.0;
+#pragma unroll
+            for (int rr = 0; rr < RG; ++rr) {
+                const int row = 16 * rr + 4 * lg;  // b is a multiple of 4
+                double f[4];
+                const bool fok = a0 + lc < rk && row < b;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[e] = fok ? Fin[(size_t)(a0 + lc) * b + row + e] : 0.0;
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    double x[4];
+                    const bool xok = 16 * cb + lc < cols && row < b;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = xok ? Xq[(size_t)(16 * cb + lc) * m + row + e] : 0.0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) tt[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[e], x[e], tt[cb], 0, 0, 0);
+                }
             }
-        }
-        __syncthreads();
-    }
-    double* Y = L.Y + (size_t)t * m * kB16;
 #pragma unroll
-    for (int q = 0; q < (BMAX * kB16 + 255) / 256; ++q) {
-        int e = threadIdx.x + q * 256;
-        if (e < b * kB16) {
-            int s = e / b, x = e % b;
-            Y[(size_t)s * m + (size_t)i * b + x] = acc[q];
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb)
+                        acc[rg][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(fo[v][rg], tt[cb][v], acc[rg][cb], 0, 0, 0);
         }
     }
+    if (w > 0)
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) red[w - 1][(rg * CB + cb) * 4 + v][lane] = acc[rg][cb][v];
+    __syncthreads();
+    if (w > 0) return;
+    double* out = TRANSPOSED ? Bout + ((size_t)L.boff[t] + c0) * m : L.Y + (size_t)t * m * kB16;
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                double r = acc[rg][cb][v];
+                for (int p = 0; p + 1 < nw; ++p) r += red[p][(rg * CB + cb) * 4 + v][lane];
+                const int row = 16 * rg + 4 * v + lg, col = 16 * cb + lc;
+                if (row < b && col < cols) out[(size_t)col * m + (size_t)o * b + row] = r;
+            }
 }
 
 // ---- direct mode: samples from on-the-fly kernel evaluations ----------------
@@ -196,7 +250,6 @@ static void pad_points(Context& c, int b, const std::vector<PadCloud>& cl, int64
 // register v of lane l at row 4v + l/16, column l%16.  Kernel evaluations
 // (exp, sqrt on the FP64 vector units) dominate, so the more dense columns a
 // sweep carries, the fewer evaluations a tile costs.
-typedef double v4d_t __attribute__((ext_vector_type(4)));
 
 // NB consecutive ARA blocks in one sweep over the tile's columns: block p of
 // the pass is Y_p[t][s*m + q] = sum_c K(x_q, x_c) Om[t][c*16NB + 16p + s],
@@ -870,61 +923,6 @@ __global__ void k_lr_commit(LrLevel L, int* flags) {
     atomicMax(&flags[1], S.k);
 }
 
-// B[t][a*m + j*b + x] = sum_i V_ij (U_ij^T Q_i), 64 Q columns per block
-template <int BMAX>
-__global__ void __launch_bounds__(256) k_lr_sampleT(LrLevel L, double* Bout) {
-    __shared__ double sV[BMAX * BMAX], sU[BMAX * BMAX], sQ[BMAX * 64], sT[BMAX * 64];
-    const int t = blockIdx.z, j = blockIdx.y, c0 = blockIdx.x * 64, b = L.b, m = L.m;
-    const int k = L.st[t].k;
-    if (c0 >= k) return;
-    const int nc = min(64, k - c0);
-    const double* Q = L.Q + (size_t)t * m * L.capQ;
-    constexpr int NACC = (BMAX * 64 + 255) / 256;
-    double acc[NACC];
-#pragma unroll
-    for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
-    for (int i = 0; i < L.bus; ++i) {
-        int64_t mo = L.first[t] + (int64_t)morton_xy((uint32_t)j, (uint32_t)i);
-        int rk = L.ranksMO[mo];
-        if (rk == 0) continue;
-        const double* U = L.UMO + (size_t)L.offMO[mo] * b;
-        const double* V = L.VMO + (size_t)L.offMO[mo] * b;
-        for (int e = threadIdx.x; e < rk * b; e += 256) { sU[e] = U[e]; sV[e] = V[e]; }
-        for (int e = threadIdx.x; e < b * nc; e += 256) {
-            int cc = e / b, x = e % b;
-            sQ[e] = Q[(size_t)(c0 + cc) * m + (size_t)i * b + x];
-        }
-        __syncthreads();
-        for (int e = threadIdx.x; e < rk * nc; e += 256) {  // sT[cc*rk + a] = U_a . Q_cc
-            int cc = e / rk, a = e % rk;
-            double v = 0.0;
-            for (int x = 0; x < b; ++x) v += sU[a * b + x] * sQ[cc * b + x];
-            sT[e] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < NACC; ++q) {
-            int e = threadIdx.x + q * 256;
-            if (e < b * nc) {
-                int cc = e / b, x = e % b;
-                double v = acc[q];
-                for (int a = 0; a < rk; ++a) v += sV[a * b + x] * sT[cc * rk + a];
-                acc[q] = v;
-            }
-        }
-        __syncthreads();
-    }
-    double* B = Bout + (size_t)L.boff[t] * m;
-#pragma unroll
-    for (int q = 0; q < NACC; ++q) {
-        int e = threadIdx.x + q * 256;
-        if (e < b * nc) {
-            int cc = e / b, x = e % b;
-            B[(size_t)(c0 + cc) * m + (size_t)j * b + x] = acc[q];
-        }
-    }
-}
-
 // grow Q capacity: copy each tile's first k columns
 __global__ void __launch_bounds__(256) k_lr_regrow(int T, int m, int oldCap, int newCap, const LrState* st,
                                                    const double* __restrict__ Qold, double* __restrict__ Qnew) {
@@ -992,17 +990,22 @@ struct LevelSource {
     int d = 0;
 };
 
-template <int BMAX>
-static void launch_sample_tlr(Context& c, const LrLevel& L, int bus, int T) {
-    k_lr_sample<BMAX><<<dim3(bus, T), 256, 0, c.stream>>>(L);
+// 16-row groups of a leaf: 1 (leaves of 8 and 16), 2 or 4
+template <int RG>
+static void launch_leaf_sum(Context& c, const LrLevel& L, int T, int kmax, double* B) {
+    const unsigned threads = 64u * (unsigned)std::min(4, L.bus);
+    if (B)
+        k_lr_leaf_sum<RG, 4, true><<<dim3((unsigned)((kmax + 63) / 64), (unsigned)L.bus, (unsigned)T), threads, 0,
+                                     c.stream>>>(L, B);
+    else
+        k_lr_leaf_sum<RG, 1, false><<<dim3(1, (unsigned)L.bus, (unsigned)T), threads, 0, c.stream>>>(L, nullptr);
     HMX_LAUNCHED();
 }
-
-template <int BMAX>
-static void launch_sampleT_tlr(Context& c, const LrLevel& L, int kmax, int bus, int T, double* B) {
-    dim3 g((unsigned)((kmax + 63) / 64), (unsigned)bus, (unsigned)T);
-    k_lr_sampleT<BMAX><<<g, 256, 0, c.stream>>>(L, B);
-    HMX_LAUNCHED();
+// the next block's samples Y = A Om, or with B the V factors A^T Q of up to kmax columns
+static void launch_sample_tlr(Context& c, const LrLevel& L, int T, int kmax = 0, double* B = nullptr) {
+    if (L.b <= 16) launch_leaf_sum<1>(c, L, T, kmax, B);
+    else if (L.b <= 32) launch_leaf_sum<2>(c, L, T, kmax, B);
+    else launch_leaf_sum<4>(c, L, T, kmax, B);
 }
 
 // direct samplers: workgroups of nw waves, all in one tile (m is 64 * 2^j)
@@ -1270,8 +1273,7 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         } else {
             k_lr_omega<<<dim3((m * kB16 + 255) / 256, T), 256, 0, c.stream>>>(L, it, 1, 0);
             HMX_LAUNCHED();
-            if (b <= 32) launch_sample_tlr<32>(c, L, bus, T);
-            else launch_sample_tlr<64>(c, L, bus, T);
+            launch_sample_tlr(c, L, T);
         }
         const unsigned kb = (unsigned)std::max(1, (kmax + 15) / 16);
         for (int pass = 0; pass < 2 && kmax > 0; ++pass) {
@@ -1378,10 +1380,8 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
                 ws.samplerFlops += 2.0 * mm * hst[t].k;
                 ws.kernelEvals += mm * (double)((hst[t].k + 63) / 64);
             }
-        } else if (b <= 32) {
-            launch_sampleT_tlr<32>(c, L, kmax, bus, T, out.V.p);
         } else {
-            launch_sampleT_tlr<64>(c, L, kmax, bus, T, out.V.p);
+            launch_sample_tlr(c, L, T, kmax, out.V.p);
         }
         dim3 g(std::min<unsigned>(1024, (unsigned)(((size_t)m * kmax + 255) / 256 + 1)), T);
         k_lr_pack<<<g, 256, 0, c.stream>>>(T, m, capQ, ws.st.p, ws.off.p, ws.Q.p, out.U.p);

@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(256) k_lr_omega(LrLevel L, int it, int nb, int
 // through LDS and no wave waits for another until the waves' sums are folded
 // in order at the end.  Bound by the latency of a leaf's loads (rank, then
 // factors: 128-byte lines) for the few tiles of the top levels, by the
-XX
+// factors' bytes below.  N = 16384 2D, all levels: 2.7 ms for A Om and
 // A^T Q together; a workgroup per leaf with factors and products staged in
 // LDS, three barriers per leaf, took 7.5.
 template <int RG, int CB, bool TRANSPOSED>

@@ -332,7 +332,7 @@ def main():
         "kernel_ms": {"phase1_VTx": ms[0], "reduce": ms[1], "phase2_Uz_Dx": ms[2], "call": ms[3]},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": traffic_bytes(args, dom),
-                     "kernel": "k_mv_phase1" if dom == 1 else "k_mv_phase2 + k_mv_phase2b",
+                     "kernel": "k_mv_phase1" if dom == 1 else "k_mv_phase2",
                      "kernel_bytes": int(dom_bytes),
                      "kernel_ms": dom_ms, "measured_read_ceiling": round(read_ceiling, 1),
                      "frac_of_measured_ceiling": round(achieved / read_ceiling, 4)},
@@ -420,8 +420,7 @@ def traffic_bytes(args, dom):
                     "_ZN3hmx11k_mf_phase1IDF16_Li4ELi4ELb1ELb0EDF16_"])
         p2 = total(["_ZN3hmx12k_mf_phase2gILi64ELb0EffDF16_Li4EfLb0E"])
         return None if p1 is None or p2 is None else (p1, p2)
-    # phase 2 is the per-leaf pass plus the tall-tile (128-row block) pass
-    return total(["k_mv_phase1<1>"] if dom == 1 else ["k_mv_phase2<64, 1>", "k_mv_phase2b<128, 1"])
+    return total(["k_mv_phase1<1>"] if dom == 1 else ["k_mv_phase2<64, 1, 4>"])
 
 
 def cpu_baseline(pipe, ctx, x1, budget_s, stride, args):

@@ -154,11 +154,17 @@ __device__ inline double lane_f64(double v, int lane) {
 // DPP step adds two values that every lane of the pair adds in either order
 // (a + b == b + a exactly), so every lane of a 16-lane row ends with the same
 // row sum; the four row sums are then added in a fixed order.
-__device__ inline double wave_sum_dpp(double v) {
+// every lane of a row of 16 gets the row's sum
+__device__ inline double row_sum_dpp(double v) {
     v += dpp_f64<0xB1>(v);
     v += dpp_f64<0x4E>(v);
     v += dpp_f64<0x141>(v);
     v += dpp_f64<0x140>(v);
+    return v;
+}
+
+__device__ inline double wave_sum_dpp(double v) {
+    v = row_sum_dpp(v);
     return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
 }
 

@@ -180,11 +180,17 @@ struct HLevel {
 
 // Phase-1 work item: a contiguous run of one tile's input-side factor
 // (V for H*x, U for H^T*x).  colLen == 0: the run is one chunk of a single
-// column (len elements, one partial result); colLen > 0: the run holds
-// len/colLen whole columns of length colLen, one result per column.
+// column (len elements); colLen > 0: the run holds len/colLen whole columns of
+// length colLen, one result per column.  out >= 0: the results are z of the
+// columns out, out + 1, ...; out < 0: the chunk's partial sum ~out of a column
+// in several chunks.
 struct MvItem {
     const double* v;
     int32_t xoff, len, colLen, out;
+};
+// A column whose z is the sum of np partial sums from part on
+struct MvSplit {
+    int32_t col, part, np;
 };
 // Phase-2 entry: the leaf's rows of one tile's output-side factor.
 struct MvEntry {
@@ -216,44 +222,34 @@ struct PlanHost {
     std::vector<NearRef> nears;     // leaf-level tiles applied as dense blocks
     uint64_t lowRankBytes = 0;      // U and V bytes of the tiles applied as factors
     std::vector<MvItem> items;
-    std::vector<int64_t> colPart;
-    std::vector<int32_t> colNpart;
+    std::vector<MvSplit> splits;    // the columns in several chunks
     std::vector<int32_t> leafPtr;   // [S+1]
     std::vector<MvEntry> entries;
-    // tiles of dimension >= rowBlock (0: none), per rowBlock-row block of the
-    // padded space instead of per leaf
-    int rowBlock = 0;
-    std::vector<int32_t> blkPtr;    // [S*b/rowBlock + 1]
-    std::vector<MvEntry> blkEntries;
     int64_t numCols = 0, numPart = 0;
 };
 
 // Per-call workspaces of the streaming matvec kernels: chunk partial sums,
-// z, and (partial leaves) x and y in the padded space.
+// z, and (partial leaves) x in the padded space.
 struct MvWork {
-    double *zpart, *z, *Xp, *Yp;
+    double *zpart, *z, *Xp;
 };
 
 // Device-side tables used by the matvec kernels (built once per H-matrix).
 struct MatvecPlan {
     DBuf<MvItem> items;
     int32_t numItems = 0;
-    DBuf<int64_t> colPart;   // per global column: first partial slot
-    DBuf<int32_t> colNpart;  // per global column: number of partial slots
+    DBuf<MvSplit> splits;    // columns in several chunks
+    int32_t numSplits = 0;
     int64_t numCols = 0, numPart = 0;
     int32_t numLeaves = 0;
     DBuf<int32_t> leafPtr;   // [S+1] CSR over leaves
     DBuf<MvEntry> entries;
-    int rowBlock = 0;        // tiles of dimension >= rowBlock in a second phase-2 pass (0: none)
-    int32_t numBlocks = 0;
     // leaf-level tiles of rank above b/2 as dense column-major b x b blocks
     int64_t numNear = 0;
     DBuf<int32_t> nearPtr, nearCol;  // CSR over output leaves; the block's input leaf
     DBuf<double> nearD;
     uint64_t bytes = 0;              // factor and dense-block bytes one pass reads
     uint64_t lowRankBytes = 0;       // of which U and V of the tiles applied as factors
-    DBuf<int32_t> blkPtr;    // CSR over rowBlock-row blocks
-    DBuf<MvEntry> blkEntries;
     const double* diag = nullptr;  // D (or D^T for the transpose plan)
     DBuf<double> diagT;            // owned transposed copy
     int chunk = 2048;              // elements of one single-column phase-1 item
@@ -263,7 +259,7 @@ struct MatvecPlan {
     bool gather = false;
     DBuf<int32_t> gmap;            // padded position -> vector index, -1 for padding
     // per-call workspaces (grown on demand)
-    DBuf<double> zpart, z, Xp, Yp;
+    DBuf<double> zpart, z, Xp;
     uint32_t wsK = 0;
 };
 
@@ -465,7 +461,7 @@ void hmatrix_save(Context& c, const HMatrix& h, const char* path);
 void hmatrix_load(Context& c, const char* path, HMatrix& h);
 void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P);
 void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const double* X, int64_t ldx, double* Xp);
-PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bool denseNear);
+PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, bool denseNear);
 void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H);
 // out[q] = A_q B_q^T, row-major b x b blocks one after the other
 void near_blocks_f64(Context& c, int b, int64_t n, const NearPair* src, double* out);
@@ -484,7 +480,6 @@ inline int mf_pass_blocks(uint32_t k) {
 uint32_t pass_width(uint32_t rem);
 void run_matvec_plan(Context& c, MatvecPlan& P, int b, uint32_t k, const double* X, int64_t ldx, double* Y,
                      hipEvent_t* ev);
-size_t matvec_ws_elems(const MatvecPlan& P, uint32_t K);
 void run_matvec_plan_ws(Context& c, const MatvecPlan& P, const MvWork& W, int b, uint32_t k, const double* X, int64_t ldx,
                         double* Y, hipEvent_t* ev);
 void build_batch_plan(Context& c, const std::vector<HMatrix*>& hs, int chunk, MatvecPlan& P, DBuf<double>& diag);

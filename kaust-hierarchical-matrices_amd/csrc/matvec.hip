@@ -7,14 +7,13 @@
 //   phase 1  z_t = V_t^T x : one wave per work item, a contiguous run of V
 //            read with 16-byte loads; long columns are split into chunks
 //            (2048 elements by default, tunable) that produce partial sums,
-//            short columns are packed many per item and reduced with segmented
-//            wave reductions;
-//   reduce   z = sum of the chunk partials (fixed order -> deterministic);
+//            short columns are packed some per item and reduced with segmented
+//            wave reductions, straight into z;
+//   reduce   z of the chunked columns = sum of their partials (fixed order ->
+//            deterministic; no launch if no column is chunked);
 //   phase 2  one workgroup per leaf (32 or 64 rows): y_leaf = D_leaf x_leaf + sum of the
-//            leaf's rows of every U_t covering it times z_t; with 64-row leaves
-//            the tiles of 128 rows and more are left to a second pass, one
-//            workgroup per 128-row block adding them to y in a fixed order.
-//            No atomics.
+//            leaf's rows of every U_t covering it times z_t, straight into the
+//            caller's entries.  No atomics.
 // The factors stay where the build left them (no per-call V transpose as in
 // src/cutlassHMatrixXVector.cu:118-150, no per-call host problem assembly).
 #include <algorithm>
@@ -24,13 +23,7 @@
 
 namespace hmx {
 
-constexpr int kRowBlock = 128;  // rows per workgroup of the tall-tile phase-2 pass
-
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
+constexpr int kPack = 512;  // elements per phase-1 item of short columns (plan_host)
 
 // factor data is read once per call: non-temporal loads keep x and z in L2
 typedef double f64x2_t __attribute__((ext_vector_type(2)));
@@ -56,7 +49,7 @@ __device__ inline void vload_d(const double* __restrict__ p, double (&out)[N]) {
 // of their arithmetic, so every lane has U loads in flight.
 template <int K>
 __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ items, int numItems,
-                                                   const double* __restrict__ X, int ldx,
+                                                   const double* __restrict__ X, int ldx, double* __restrict__ z,
                                                    double* __restrict__ zpart) {
     constexpr int U = K <= 4 ? 4 : (K == 8 ? 2 : 1);  // keep the register file for occupancy at wide K
     const int lane = threadIdx.x & 63;
@@ -68,6 +61,7 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
     const int len = it.len;
     const int m = it.colLen ? it.colLen : len;  // column length inside this item (power of two)
     const double* __restrict__ xs = X + it.xoff;
+    double* __restrict__ out = it.out >= 0 ? z + (size_t)it.out * K : zpart + (size_t)~it.out * K;
     if (m == 128) {
         // one column per step, and a lane meets the same two x entries in every step
         double2 xr[K];
@@ -82,14 +76,14 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
                                            : make_double2(0.0, 0.0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (e0 + 128 * u >= len) break;
+                // the sums of U columns side by side (no branch between them)
 #pragma unroll
                 for (int s = 0; s < K; ++s) {
-                    const double r = wave_sum(fma(vv[u].y, xr[s].y, vv[u].x * xr[s].x));
-                    if (lane == 0) zpart[(size_t)(it.out + col) * K + s] = r;
+                    const double r = wave_sum_dpp(fma(vv[u].y, xr[s].y, vv[u].x * xr[s].x));
+                    if (lane == 0 && e0 + 128 * u < len) out[(size_t)(col + u) * K + s] = r;
                 }
-                ++col;
             }
+            col += U;
         }
     } else if (m > 128) {
         // every 128-element step lies inside one column
@@ -120,8 +114,8 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
                 if (((e0 + 128 * u + 128) & (m - 1)) == 0) {
 #pragma unroll
                     for (int s = 0; s < K; ++s) {
-                        const double r = wave_sum(acc[s]);
-                        if (lane == 0) zpart[(size_t)(it.out + col) * K + s] = r;
+                        const double r = wave_sum_dpp(acc[s]);
+                        if (lane == 0) out[(size_t)col * K + s] = r;
                         acc[s] = 0.0;
                     }
                     ++col;
@@ -145,18 +139,17 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (e0 + 128 * u >= len) break;
                 const int e = e0 + 128 * u + 2 * lane;
                 double p[K];
 #pragma unroll
-                for (int s = 0; s < K; ++s) p[s] = fma(vv[u].y, xr[s].y, vv[u].x * xr[s].x);
-                for (int off = 1; off < g; off <<= 1)
-#pragma unroll
-                    for (int s = 0; s < K; ++s) p[s] += __shfl_xor(p[s], off, 64);
+                for (int s = 0; s < K; ++s) {
+                    p[s] = row_sum_dpp(fma(vv[u].y, xr[s].y, vv[u].x * xr[s].x));
+                    if (m == 64) p[s] += __shfl_xor(p[s], 16, 64);
+                }
                 if (e < len && (lane & (g - 1)) == 0) {
                     const int col = e / m;
 #pragma unroll
-                    for (int s = 0; s < K; ++s) zpart[(size_t)(it.out + col) * K + s] = p[s];
+                    for (int s = 0; s < K; ++s) out[(size_t)col * K + s] = p[s];
                 }
             }
         }
@@ -164,37 +157,51 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
 }
 
 // ---- reduce partials ---------------------------------------------------------
-__global__ void __launch_bounds__(256) k_mv_reduce(int64_t numCols, int K, const int64_t* __restrict__ colPart,
-                                                   const int32_t* __restrict__ colNpart,
+// (only the columns in several chunks: phase 1 wrote z of the others)
+__global__ void __launch_bounds__(256) k_mv_reduce(int numSplits, int K, const MvSplit* __restrict__ splits,
                                                    const double* __restrict__ zpart, double* __restrict__ z) {
-    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= numCols * K) return;
-    int64_t g = e / K;
-    int s = (int)(e % K);
-    const int64_t p0 = colPart[g];
-    const int np = colNpart[g];
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (int64_t)numSplits * K) return;
+    const MvSplit sp = splits[e / K];
+    const int s = (int)(e % K);
     double v = 0.0;
-    for (int c = 0; c < np; ++c) v += zpart[(p0 + c) * K + s];
-    z[e] = v;
+    for (int c = 0; c < sp.np; ++c) v += zpart[((size_t)sp.part + c) * K + s];
+    z[(size_t)sp.col * K + s] = v;
 }
 
 // ---- phase 2 -----------------------------------------------------------------
 // 256 threads = 16 column groups x 16 lanes; a lane owns RPL = BL/16
 // consecutive rows of the leaf (BL = bucketSize) and a column group walks
-// columns cg, cg+16, ...
-template <int BL, int K>
-__global__ void __launch_bounds__(256) k_mv_phase2(const int32_t* __restrict__ leafPtr,
+// columns cg, cg+16, ...  Bound by HBM at large n and by the chain of a leaf's
+// blocks and tiles (one round trip each) at small n: with one right-hand side,
+// where the registers leave room, mv_parts = 4 such groups of threads take
+// every fourth block and tile, each group a sum of its own, the sums added in
+// a fixed order.  The number of parts hangs on K alone, never on the plan, so
+// that a batch and its instances sum alike.  Measured, phase 2 of one
+// right-hand side, 1 part -> 4: N = 1000 / 4096 / 16384 / 65536 / 200000 2D
+// 12.4 / 27.9 / 47.6 / 115 / 478 us -> 7.6 / 12.0 / 25.9 / 105 / 457.  4
+// right-hand sides at N = 65536 2D: 155 us -> 165, 8 (2 parts) 218 -> 260: one
+// part there.  All tiles go here, tall ones too: a second pass over row blocks
+// of 128 for tiles of 128 rows and more (64-row leaves; before the parts the
+// faster way at N = 2^20, 14.9 -> 13.0 ms) takes 45.5 / 112 / 502 / 1162 us at
+// N = 4096 / 16384 / 60000 / 120000 3D, this kernel alone 33.0 / 100 / 487 /
+// 1103, and at N = 2^20 14.3 ms both.
+constexpr int mv_parts(int K) { return K == 1 ? 4 : 1; }
+template <int BL, int K, int NS = mv_parts(K)>
+__global__ void __launch_bounds__(256 * NS) k_mv_phase2(const int32_t* __restrict__ leafPtr,
                                                    const MvEntry* __restrict__ entries,
                                                    const double* __restrict__ diag, const double* __restrict__ z,
                                                    const double* __restrict__ X, int ldx, double* __restrict__ Y,
+                                                   int64_t ldy, const int32_t* __restrict__ gmap,
                                                    const int32_t* __restrict__ nearPtr,
                                                    const int32_t* __restrict__ nearCol,
                                                    const double* __restrict__ nearD) {
     constexpr int RPL = BL / 16;
     static_assert(RPL == 2 || RPL == 4, "bucketSize 32 or 64");
-    __shared__ double red[4][BL * K];
+    __shared__ double red[4 * NS][BL * K];
     const int leaf = blockIdx.x;
-    const int l16 = threadIdx.x & 15, cg = threadIdx.x >> 4;
+    const int l16 = threadIdx.x & 15, cg = (threadIdx.x >> 4) & 15;
+    const int part = NS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     // lane l16 holds rows 2*l16 + {0, 1} (+ 32 for its second pair with
     // 64-row leaves): each 16-byte load instruction of a column reads 256
     // contiguous bytes (a lane reading 4 consecutive rows as two loads used
@@ -220,7 +227,7 @@ __global__ void __launch_bounds__(256) k_mv_phase2(const int32_t* __restrict__ l
     // dense blocks (column-major): the diagonal block, then the leaf's
     // near-field blocks; columns c = cg, cg+16, ... of each
     const int q0 = nearPtr ? nearPtr[leaf] : 0, q1 = nearPtr ? nearPtr[leaf + 1] : 0;
-    for (int q = q0 - 1; q < q1; ++q) {
+    for (int q = q0 - 1 + part; q < q1; q += NS) {
         const double* D = q < q0 ? diag + (size_t)leaf * BL * BL : nearD + (size_t)q * BL * BL;
         const double* xl = X + (size_t)(q < q0 ? leaf : nearCol[q]) * BL;
 #pragma unroll
@@ -237,7 +244,7 @@ __global__ void __launch_bounds__(256) k_mv_phase2(const int32_t* __restrict__ l
         }
     }
     const int e0 = leafPtr[leaf], e1 = leafPtr[leaf + 1];
-    for (int e = e0; e < e1; ++e) {
+    for (int e = e0 + part; e < e1; e += NS) {
         const MvEntry en = entries[e];
         const double* __restrict__ U = en.u;
         const double* __restrict__ zz = z + (size_t)en.zbase * K;
@@ -280,71 +287,13 @@ __global__ void __launch_bounds__(256) k_mv_phase2(const int32_t* __restrict__ l
 #pragma unroll
             for (int q = 0; q < RPL; ++q) red[wave][s * BL + rowq(q)] = acc[q][s];
     __syncthreads();
-    for (int o = threadIdx.x; o < BL * K; o += 256) {
-        const double v = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
+    for (int o = threadIdx.x; o < BL * K; o += 256 * NS) {
+        double v = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
+#pragma unroll
+        for (int t = 4; t < 4 * NS; t += 4) v += (red[t][o] + red[t + 1][o]) + (red[t + 2][o] + red[t + 3][o]);
         const int s = o / BL, row = o % BL;
-        Y[(size_t)s * ldx + (size_t)leaf * BL + row] = v;
-    }
-}
-
-// ---- phase 2, tall tiles ------------------------------------------------------
-// One workgroup per block of RB rows adds the tiles of dimension >= RB to y
-// (after the per-leaf pass wrote it).  Every wave covers all RB rows, RPL =
-// RB/64 consecutive rows per lane, so one column's segment is one contiguous
-// RB*8-byte read (the per-leaf pass reads 512-byte pieces of the same columns
-// at m*8-byte strides); wave w takes columns w, w+4, ..., CPS of them per
-// step.  Blocks are numbered XCD-locally: the blocks of one tall tile share
-// its z and meet in one L2.  The four waves' partial sums are folded in LDS
-// in a fixed order.
-template <int RB, int K, int CPS = 4>
-__global__ void __launch_bounds__(256) k_mv_phase2b(const int32_t* __restrict__ blkPtr,
-                                                    const MvEntry* __restrict__ entries,
-                                                    const double* __restrict__ z, double* __restrict__ Y, int ldy) {
-    constexpr int RPL = RB / 64;
-    static_assert(RPL % 2 == 0, "16-byte loads");
-    __shared__ double red[4][RB];
-    const int blk = xcd_local(blockIdx.x, gridDim.x);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r0 = RPL * lane;
-    double acc[RPL][K];
-#pragma unroll
-    for (int q = 0; q < RPL; ++q)
-#pragma unroll
-        for (int s = 0; s < K; ++s) acc[q][s] = 0.0;
-    const int e0 = blkPtr[blk], e1 = blkPtr[blk + 1];
-    for (int e = e0; e < e1; ++e) {
-        const MvEntry en = entries[e];
-        const double* __restrict__ U = en.u;
-        const double* __restrict__ zz = z + (size_t)en.zbase * K;
-        for (int j0 = w; j0 < en.rank; j0 += 4 * CPS) {
-            double u[CPS][RPL], zv[CPS][K];
-#pragma unroll
-            for (int p = 0; p < CPS; ++p) {
-                const int j = j0 + 4 * p;
-                if (j < en.rank) {
-                    vload_d<RPL>(U + (size_t)j * en.m + r0, u[p]);
-#pragma unroll
-                    for (int s = 0; s < K; ++s) zv[p][s] = zz[(size_t)j * K + s];
-                }
-            }
-#pragma unroll
-            for (int p = 0; p < CPS; ++p)
-                if (j0 + 4 * p < en.rank)
-#pragma unroll
-                    for (int s = 0; s < K; ++s)
-#pragma unroll
-                        for (int q = 0; q < RPL; ++q) acc[q][s] = fma(u[p][q], zv[p][s], acc[q][s]);
-        }
-    }
-    double* __restrict__ Yb = Y + (size_t)blk * RB;
-#pragma unroll
-    for (int s = 0; s < K; ++s) {
-#pragma unroll
-        for (int q = 0; q < RPL; ++q) red[w][r0 + q] = acc[q][s];
-        __syncthreads();
-        for (int row = threadIdx.x; row < RB; row += 256)
-            Yb[(size_t)s * ldy + row] += (red[0][row] + red[1][row]) + (red[2][row] + red[3][row]);
-        __syncthreads();
+        const int64_t pos = (int64_t)leaf * BL + row, i = gmap ? gmap[pos] : pos;  // -1 on padding
+        if (i >= 0) Y[(size_t)s * ldy + i] = v;
     }
 }
 
@@ -359,7 +308,7 @@ __global__ void __launch_bounds__(256) k_transpose_blocks(int S, int b, const do
     DT[leaf * per + (int64_t)q * b + c] = D[e];
 }
 
-// vectors (ldx apart) <-> the padded space (npad apart), K right-hand sides
+// vectors (ldx apart) to the padded space (npad apart), K right-hand sides
 __global__ void __launch_bounds__(256) k_gather(int64_t npad, int K, const int32_t* __restrict__ gmap,
                                                 const double* __restrict__ X, int64_t ldx, double* __restrict__ Xp) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -369,27 +318,16 @@ __global__ void __launch_bounds__(256) k_gather(int64_t npad, int K, const int32
     Xp[e] = g >= 0 ? X[s * ldx + g] : 0.0;
 }
 
-__global__ void __launch_bounds__(256) k_scatter(int64_t npad, int K, const int32_t* __restrict__ gmap,
-                                                 const double* __restrict__ Yp, double* __restrict__ Y, int64_t ldy) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= npad * K) return;
-    const int64_t s = e / npad, p = e % npad;
-    const int g = gmap[p];
-    if (g >= 0) Y[s * ldy + g] = Yp[e];
-}
-
 // Work lists of one H-matrix: phase-1 items over the input-side factors,
 // partial-slot bookkeeping, phase-2 entries per output leaf.  Positions are
 // in the padded space (leaf*b + i).
-PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bool denseNear) {
+PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, bool denseNear) {
     const int L = h.numLevels, b = (int)h.b, S = (int)h.S;
     HMX_CHECK(b == 32 || b == 64, HMX_EUNSUPPORTED, "HMatrixVecMult kernels are built for bucketSize 32 or 64");
     HMX_CHECK(chunk >= 128 && (chunk & (chunk - 1)) == 0, HMX_EINVAL, "phase-1 chunk must be a power of two >= 128");
     PlanHost H;
     H.b = b;
     std::vector<std::vector<MvEntry>> leafEntries(S);
-    const int nblk = rowBlock > 0 ? (int)((int64_t)S * b / rowBlock) : 0;
-    std::vector<std::vector<MvEntry>> blkEntries(nblk);
     int64_t slot = 0, g = 0;
     for (int l = 1; l < L; ++l) {
         const HLevel& lv = h.levels[l - 1];
@@ -409,31 +347,28 @@ PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bo
             }
             H.lowRankBytes += 16ull * (uint64_t)r * (uint64_t)m;
             const int nch = m >= chunk ? m / chunk : 1;
-            for (int j = 0; j < r; ++j) {
-                H.colPart.push_back(slot + (int64_t)j * nch);
-                H.colNpart.push_back(nch);
-            }
-            if (m >= chunk) {
-                for (int j = 0; j < r; ++j)
+            if (nch > 1) {
+                for (int j = 0; j < r; ++j) {
+                    H.splits.push_back(MvSplit{(int32_t)(g + j), (int32_t)(slot + (int64_t)j * nch), nch});
                     for (int q = 0; q < nch; ++q)
                         H.items.push_back(MvItem{Pin + (size_t)j * m + (size_t)q * chunk, (int32_t)(inCl * m + q * chunk),
-                                                 chunk, 0, (int32_t)(slot + (int64_t)j * nch + q)});
+                                                 chunk, 0, ~(int32_t)(slot + (int64_t)j * nch + q)});
+                }
+                slot += (int64_t)r * nch;
             } else {
-                const int cpi = chunk / m;
+                // short columns: kPack elements per item, or one column (a
+                // wave reduces its columns one after the other; phase 1 of
+                // N = 4096 / 16384 / 65536 / 200000 2D with items of 'chunk'
+                // elements 9.4 / 20.0 / 82.4 / 417 us, of 512 6.5 / 17.2 /
+                // 80.5 / 409, of 256 6.6 / 17.9 / 83.3 / 419)
+                const int cpi = std::max(1, std::min(chunk, kPack) / m);
                 for (int j0 = 0; j0 < r; j0 += cpi) {
                     const int nc = std::min(cpi, r - j0);
-                    H.items.push_back(MvItem{Pin + (size_t)j0 * m, (int32_t)(inCl * m), nc * m, m, (int32_t)(slot + j0)});
+                    H.items.push_back(MvItem{Pin + (size_t)j0 * m, (int32_t)(inCl * m), nc * m, m, (int32_t)(g + j0)});
                 }
             }
-            if (rowBlock > 0 && m >= rowBlock) {
-                const int nb = m / rowBlock;
-                for (int q = 0; q < nb; ++q)
-                    blkEntries[outCl * nb + q].push_back(MvEntry{Pout + (size_t)q * rowBlock, m, r, (int32_t)g, 0});
-            } else {
-                for (int q = 0; q < bus; ++q)
-                    leafEntries[outCl * bus + q].push_back(MvEntry{Pout + (size_t)q * b, m, r, (int32_t)g, 0});
-            }
-            slot += (int64_t)r * nch;
+            for (int q = 0; q < bus; ++q)
+                leafEntries[outCl * bus + q].push_back(MvEntry{Pout + (size_t)q * b, m, r, (int32_t)g, 0});
             g += r;
         }
     }
@@ -444,15 +379,6 @@ PlanHost plan_host(const HMatrix& h, bool transpose, int chunk, int rowBlock, bo
         H.entries.insert(H.entries.end(), leafEntries[leaf].begin(), leafEntries[leaf].end());
     }
     H.leafPtr[S] = (int32_t)H.entries.size();
-    H.rowBlock = nblk > 0 ? rowBlock : 0;
-    if (nblk > 0) {
-        H.blkPtr.assign(nblk + 1, 0);
-        for (int k = 0; k < nblk; ++k) {
-            H.blkPtr[k] = (int32_t)H.blkEntries.size();
-            H.blkEntries.insert(H.blkEntries.end(), blkEntries[k].begin(), blkEntries[k].end());
-        }
-        H.blkPtr[nblk] = (int32_t)H.blkEntries.size();
-    }
     H.numCols = g;
     H.numPart = slot;
     return H;
@@ -470,16 +396,10 @@ void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H) {
     P.numPart = H.numPart;
     P.numLeaves = (int32_t)H.leafPtr.size() - 1;
     put(c, P.items, H.items);
-    put(c, P.colPart, H.colPart);
-    put(c, P.colNpart, H.colNpart);
+    P.numSplits = (int32_t)H.splits.size();
+    put(c, P.splits, H.splits);
     put(c, P.leafPtr, H.leafPtr);
     put(c, P.entries, H.entries);
-    P.rowBlock = H.rowBlock;
-    P.numBlocks = H.rowBlock ? (int32_t)H.blkPtr.size() - 1 : 0;
-    if (H.rowBlock) {
-        put(c, P.blkPtr, H.blkPtr);
-        put(c, P.blkEntries, H.blkEntries);
-    }
     // dense near-field blocks, grouped by output leaf
     const int S = P.numLeaves, b = H.b;
     std::vector<NearRef> nears = H.nears;
@@ -518,15 +438,6 @@ std::vector<int32_t> padding_map(const HMatrix& h, int64_t base) {
     return gm;
 }
 
-// 64-row leaves: tiles of 128 rows and more go through the row-block pass of
-// phase 2 (measured at N = 2^20, 3D: phase 2 14.9 -> 13.0 ms; blocks of 256
-// rows 14.4 ms, of 64 rows 14.9 ms).  32-row leaves and batches: per-leaf
-// pass only.
-int row_block(const HMatrix& h) {
-    const int64_t npad = (int64_t)h.S * h.b;
-    return h.b == 64 && npad >= kRowBlock && npad % kRowBlock == 0 ? kRowBlock : 0;
-}
-
 void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const double* X, int64_t ldx, double* Xp) {
     const int64_t tot = npad * K;
     k_gather<<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(npad, K, gmap, X, ldx, Xp);
@@ -536,7 +447,7 @@ void gather_padded(Context& c, int64_t npad, int K, const int32_t* gmap, const d
 void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P) {
     const int b = (int)h.b, S = (int)h.S;
     HMX_CHECK(h.leafOffsets.size() == (size_t)S + 1, HMX_ESTATE, "H-matrix without leaf offsets");
-    upload_plan(c, P, plan_host(h, transpose, P.chunk, row_block(h), h.planDenseNear != 0));
+    upload_plan(c, P, plan_host(h, transpose, P.chunk, h.planDenseNear != 0));
     P.n = h.n;
     P.npad = (int64_t)S * b;
     P.gather = h.n != (uint32_t)P.npad;
@@ -559,34 +470,29 @@ void build_matvec_plan(Context& c, HMatrix& h, bool transpose, MatvecPlan& P) {
 
 template <int K>
 static void run_phases(Context& c, const MatvecPlan& P, const MvWork& W, int b, const double* X, int64_t ldx, double* Y,
-                       hipEvent_t* ev) {
+                       int64_t ldy, hipEvent_t* ev) {
     if (ev) HMX_HIP(hipEventRecord(ev[0], c.stream));
     if (P.numItems > 0) {
         k_mv_phase1<K><<<(unsigned)((P.numItems + 3) / 4), 256, 0, c.stream>>>(P.items.p, P.numItems, X, (int)ldx,
-                                                                                 W.zpart);
+                                                                                 W.z, W.zpart);
         HMX_LAUNCHED();
     }
     if (ev) HMX_HIP(hipEventRecord(ev[1], c.stream));
-    if (P.numCols > 0) {
-        k_mv_reduce<<<(unsigned)((P.numCols * K + 255) / 256), 256, 0, c.stream>>>(P.numCols, K, P.colPart.p,
-                                                                                   P.colNpart.p, W.zpart, W.z);
+    if (P.numSplits > 0) {
+        k_mv_reduce<<<(unsigned)(((int64_t)P.numSplits * K + 255) / 256), 256, 0, c.stream>>>(P.numSplits, K, P.splits.p,
+                                                                                              W.zpart, W.z);
         HMX_LAUNCHED();
     }
     if (ev) HMX_HIP(hipEventRecord(ev[2], c.stream));
     const int32_t* near = P.numNear ? P.nearPtr.p : nullptr;
+    const int32_t* gm = P.gather ? P.gmap.p : nullptr;  // X is padded, Y the caller's
     if (b == 64)
-        k_mv_phase2<64, K><<<(unsigned)P.numLeaves, 256, 0, c.stream>>>(P.leafPtr.p, P.entries.p, P.diag, W.z, X,
-                                                                         (int)ldx, Y, near, P.nearCol.p, P.nearD.p);
+        k_mv_phase2<64, K><<<(unsigned)P.numLeaves, 256 * mv_parts(K), 0, c.stream>>>(P.leafPtr.p, P.entries.p, P.diag, W.z, X,
+                                                                         (int)ldx, Y, ldy, gm, near, P.nearCol.p, P.nearD.p);
     else
-        k_mv_phase2<32, K><<<(unsigned)P.numLeaves, 256, 0, c.stream>>>(P.leafPtr.p, P.entries.p, P.diag, W.z, X,
-                                                                         (int)ldx, Y, near, P.nearCol.p, P.nearD.p);
+        k_mv_phase2<32, K><<<(unsigned)P.numLeaves, 256 * mv_parts(K), 0, c.stream>>>(P.leafPtr.p, P.entries.p, P.diag, W.z, X,
+                                                                         (int)ldx, Y, ldy, gm, near, P.nearCol.p, P.nearD.p);
     HMX_LAUNCHED();
-    if (P.numBlocks > 0) {  // after the per-leaf pass: it adds to Y
-        HMX_CHECK(P.rowBlock == kRowBlock, HMX_ESTATE, "matvec plan with an unknown row block");
-        k_mv_phase2b<kRowBlock, K><<<(unsigned)P.numBlocks, 256, 0, c.stream>>>(P.blkPtr.p, P.blkEntries.p, W.z,
-                                                                                 Y, (int)ldx);
-        HMX_LAUNCHED();
-    }
     if (ev) HMX_HIP(hipEventRecord(ev[3], c.stream));
 }
 
@@ -596,17 +502,14 @@ bool ensure_matvec_ws(MatvecPlan& P, uint32_t K) {
     if (P.wsK >= K) return false;
     P.zpart.alloc((size_t)std::max<int64_t>(1, P.numPart) * K);
     P.z.alloc((size_t)std::max<int64_t>(1, P.numCols) * K);
-    if (P.gather) {
-        P.Xp.alloc((size_t)P.npad * K);
-        P.Yp.alloc((size_t)P.npad * K);
-    }
+    if (P.gather) P.Xp.alloc((size_t)P.npad * K);
     P.wsK = K;
     return true;
 }
 
 // K = kernel width (1, 4, 8 or 16); k (a multiple of K) right-hand sides in
-// passes of K.  With partial leaves every pass gathers into and scatters from
-// the padded space.
+// passes of K.  With partial leaves every pass gathers X into the padded
+// space; phase 2 writes the caller's entries.
 template <int K>
 static void run_k(Context& c, const MatvecPlan& P, const MvWork& W, int b, uint32_t k, const double* X, int64_t ldx,
                   double* Y, hipEvent_t* ev) {
@@ -614,25 +517,15 @@ static void run_k(Context& c, const MatvecPlan& P, const MvWork& W, int b, uint3
         const double* Xs = X + (size_t)s0 * ldx;
         double* Ys = Y + (size_t)s0 * ldx;
         if (!P.gather) {
-            run_phases<K>(c, P, W, b, Xs, ldx, Ys, ev);
+            run_phases<K>(c, P, W, b, Xs, ldx, Ys, ldx, ev);
             continue;
         }
-        const int64_t tot = P.npad * K;
         gather_padded(c, P.npad, K, P.gmap.p, Xs, ldx, W.Xp);
-        run_phases<K>(c, P, W, b, W.Xp, P.npad, W.Yp, ev);
-        k_scatter<<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(P.npad, K, P.gmap.p, W.Yp, Ys, ldx);
-        HMX_LAUNCHED();
+        run_phases<K>(c, P, W, b, W.Xp, P.npad, Ys, ldx, ev);
     }
 }
 
 uint32_t pass_width(uint32_t rem) { return rem >= 16 ? 16 : (rem >= 8 ? 8 : (rem >= 4 ? 4 : 1)); }
-
-// Workspace elements (doubles) of passes of up to K right-hand sides:
-// partial sums, z, and with partial leaves the padded copies of x and y.
-size_t matvec_ws_elems(const MatvecPlan& P, uint32_t K) {
-    return ((size_t)std::max<int64_t>(1, P.numPart) + (size_t)std::max<int64_t>(1, P.numCols) +
-            (P.gather ? 2 * (size_t)P.npad : 0)) * K;
-}
 
 // Any k: the widest kernels first (k = 21 runs 16 + 4 + 1 right-hand sides),
 // on the workspaces W (sized for passes of pass_width(k) right-hand sides).
@@ -656,7 +549,7 @@ void run_matvec_plan_ws(Context& c, const MatvecPlan& P, const MvWork& W, int b,
 void run_matvec_plan(Context& c, MatvecPlan& P, int b, uint32_t k, const double* X, int64_t ldx, double* Y,
                      hipEvent_t* ev) {
     ensure_matvec_ws(P, pass_width(k));
-    const MvWork W{P.zpart.p, P.z.p, P.Xp.p, P.Yp.p};
+    const MvWork W{P.zpart.p, P.z.p, P.Xp.p};
     run_matvec_plan_ws(c, P, W, b, k, X, ldx, Y, ev);
 }
 
@@ -708,14 +601,14 @@ void build_batch_plan(Context& c, const std::vector<HMatrix*>& hs, int chunk, Ma
     for (HMatrix* h : hs) {
         HMX_CHECK(h->b == (uint32_t)b, HMX_EINVAL, "all instances of a batch need the same bucketSize");
         HMX_CHECK(h->leafOffsets.size() == (size_t)h->S + 1, HMX_ESTATE, "H-matrix without leaf offsets");
-        PlanHost H = plan_host(*h, false, chunk, 0, h->planDenseNear != 0);
+        PlanHost H = plan_host(*h, false, chunk, h->planDenseNear != 0);
         for (MvItem it : H.items) {
             it.xoff = (int32_t)(it.xoff + padBase);
-            it.out = (int32_t)(it.out + slotBase);
+            it.out = it.out >= 0 ? (int32_t)(it.out + colBase) : ~(int32_t)(~it.out + slotBase);
             B.items.push_back(it);
         }
-        for (int64_t p : H.colPart) B.colPart.push_back(p + slotBase);
-        B.colNpart.insert(B.colNpart.end(), H.colNpart.begin(), H.colNpart.end());
+        for (const MvSplit& sp : H.splits)
+            B.splits.push_back(MvSplit{(int32_t)(sp.col + colBase), (int32_t)(sp.part + slotBase), sp.np});
         const int32_t e0 = (int32_t)B.entries.size();
         for (MvEntry en : H.entries) {
             en.zbase = (int32_t)(en.zbase + colBase);

@@ -66,13 +66,17 @@ void hmatvec_noalloc(Context& c, const HMatrix& h, uint32_t k, const double* X, 
     const size_t nPart = round_up((size_t)std::max<int64_t>(1, P.numPart) * K);
     const size_t nZ = round_up((size_t)std::max<int64_t>(1, P.numCols) * K);
     const size_t nPad = P.gather ? round_up((size_t)P.npad * K) : 0;
-    const size_t need = (nPart + nZ + 2 * nPad) * sizeof(double);
+    // the limit counts a partial slot for every column, split or not, and y
+    // padded like x: an H-matrix is taken or refused by its sizes alone,
+    // whatever part of that the kernels keep in registers
+    const size_t nSlots = round_up((size_t)std::max<int64_t>(1, P.numPart + P.numCols - P.numSplits) * K);
+    const size_t need = (nSlots + nZ + 2 * nPad) * sizeof(double);
     HMX_CHECK(need <= kScratchBytes, HMX_EINVAL,
               "the no-allocation H-matvec needs " + std::to_string(need >> 20) + " MiB of scratch for passes of " +
                   std::to_string(K) + " right-hand sides of this H-matrix; its fixed array holds " +
                   std::to_string(kScratchBytes >> 20) + " MiB");
     double* s = static_cast<double*>(base);
-    MvWork W{s, s + nPart, P.gather ? s + nPart + nZ : nullptr, P.gather ? s + nPart + nZ + nPad : nullptr};
+    MvWork W{s, s + nPart, P.gather ? s + nPart + nZ : nullptr};
     run_matvec_plan_ws(c, P, W, (int)h.b, k, X, (int64_t)h.n, Y, nullptr);
 }
 

@@ -68,6 +68,7 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_grad_tiles(const GradItem* 
     const GradItem it = items[id];
     const int m = it.m, ncols = it.ncols;
     const int step = tall ? 16 * NW : 16, first = tall ? 16 * w : 0;
+    const double *V = in_global<double>(it.V), *U = in_global<double>(it.U);
     const double* __restrict__ Xc = X + it.colStart;
     const double* __restrict__ Wr = W + it.rowStart;
     v4d zt[CG][NB], gt[CG][NB];
@@ -84,8 +85,8 @@ __global__ void __launch_bounds__(64 * kGradWaves) k_grad_tiles(const GradItem* 
 #pragma unroll
         for (int g = 0; g < CG; ++g) {
             if (16 * g + lc < ncols) {
-                ld4(it.V + (size_t)(16 * g + lc) * m + r, vb[g]);
-                ld4(it.U + (size_t)(16 * g + lc) * m + r, ub[g]);
+                ld4(V + (size_t)(16 * g + lc) * m + r, vb[g]);
+                ld4(U + (size_t)(16 * g + lc) * m + r, ub[g]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) vb[g][e] = ub[g][e] = 0.0;

@@ -16,6 +16,19 @@ constexpr uint32_t kTagPoints = 0x504F0000u;
 constexpr uint32_t kTagOmega = 0x4F4D0000u;
 constexpr uint32_t kTagRhs = 0x52480000u;
 
+// An address read from a table in memory, of device memory.  Kernel arguments
+// are known to be such, addresses in tables are not: they are read with flat
+// loads, which count as LDS operations too, so that every wait for a table
+// entry or an LDS read waits for them as well and none stays in flight
+// behind it.  16 right-hand sides: FP64 N = 120000 3D 2405 -> 2319 us, mixed 799
+// -> 768; phase 1 of one right-hand side 746 -> 728.  Its phase 2 keeps the
+// table's address as it is (N = 65536 2D 105 us, this way 113): it has no other
+// loads to wait for.
+template <class T>
+__device__ inline const T* in_global(const void* p) {
+    return (const T*)(const __attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+
 __host__ __device__ inline void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {

@@ -61,6 +61,7 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
     const int len = it.len;
     const int m = it.colLen ? it.colLen : len;  // column length inside this item (power of two)
     const double* __restrict__ xs = X + it.xoff;
+    const double* __restrict__ v = in_global<double>(it.v);
     double* __restrict__ out = it.out >= 0 ? z + (size_t)it.out * K : zpart + (size_t)~it.out * K;
     if (m == 128) {
         // one column per step, and a lane meets the same two x entries in every step
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
             double2 vv[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                vv[u] = e0 + 128 * u < len ? ld_nt2(it.v + e0 + 128 * u + 2 * lane)
+                vv[u] = e0 + 128 * u < len ? ld_nt2(v + e0 + 128 * u + 2 * lane)
                                            : make_double2(0.0, 0.0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -97,7 +98,7 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
             for (int u = 0; u < U; ++u) {
                 const int e = e0 + 128 * u + 2 * lane;
                 const bool ok = e0 + 128 * u < len;  // uniform: len is a multiple of 128
-                vv[u] = ok ? ld_nt2(it.v + e) : make_double2(0.0, 0.0);
+                vv[u] = ok ? ld_nt2(v + e) : make_double2(0.0, 0.0);
                 const int xi = e & (m - 1);
 #pragma unroll
                 for (int s = 0; s < K; ++s)
@@ -135,7 +136,7 @@ __global__ void __launch_bounds__(256) k_mv_phase1(const MvItem* __restrict__ it
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int e = e0 + 128 * u + 2 * lane;
-                vv[u] = e < len ? ld_nt2(it.v + e) : make_double2(0.0, 0.0);
+                vv[u] = e < len ? ld_nt2(v + e) : make_double2(0.0, 0.0);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {

@@ -170,6 +170,7 @@ __device__ inline size_t xb_index(int64_t row, int s, int sh) {
 // double buffer (29.6 against 32.9 us with 4).
 constexpr int kPipe = 4;   // phase 2
 constexpr int kPipe1 = 2;  // phase 1
+constexpr int kP2Chunk = 8;  // phase2_grid
 
 // ---- phase 1 ---------------------------------------------------------------
 // SPLIT (T = FP16): the FP32 group of a mixed plan with V held as FP16 hi +
@@ -217,7 +218,7 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     using ACC = typename M::acc_t;
     const MfItem it = items[wid];
     if (16 * g0 >= it.ncols) return;
-    const T* __restrict__ V = (const T*)it.v;
+    const T* __restrict__ V = in_global<T>(it.v);
     typename M::accv acc[CG][NB];
 #pragma unroll
     for (int g = 0; g < CG; ++g)
@@ -528,12 +529,12 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
 #pragma unroll
             for (int rg = 0; rg < RG; ++rg) {
                 if (UCM) {  // column-major U in place: one element per column, zero past the rank
-                    const T* U = (const T*)en.u + rowOff + 16 * rg + lc;
+                    const T* U = in_global<T>(en.u) + rowOff + 16 * rg + lc;
 #pragma unroll
                     for (int q = 0; q < VL; ++q)
                         A[rg][q] = cc + q < en.rank ? __builtin_nontemporal_load(U + (size_t)(cc + q) * en.ld) : (T)0;
                 } else {
-                    const T* U = (const T*)en.u + (size_t)(rowOff / 16 + rg) * 16 * en.rpad + (size_t)16 * c0 +
+                    const T* U = in_global<T>(en.u) + (size_t)(rowOff / 16 + rg) * 16 * en.rpad + (size_t)16 * c0 +
                                  (16 * lg + lc) * E16;
 #pragma unroll
                     for (int p = 0; p < NP; ++p) vload16_nt(U + p * pstride, &A[rg][p * E16]);
@@ -655,7 +656,7 @@ __device__ inline void lr_rows_split(const MfEntry* __restrict__ ents, int e0, i
                 const int pstride = 16 * E16 * (min(SS, en.rpad - c0) / VL);
 #pragma unroll
                 for (int rg = 0; rg < RG; ++rg) {
-                    const _Float16* U = (const _Float16*)en.u + (size_t)(rowOff / 16 + rg) * 16 * en.rpad +
+                    const _Float16* U = in_global<_Float16>(en.u) + (size_t)(rowOff / 16 + rg) * 16 * en.rpad +
                                         (size_t)16 * c0 + (16 * lg + lc) * E16;
 #pragma unroll
                     for (int p = 0; p < NP; ++p) {
@@ -734,7 +735,7 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
     auto dload = [&](int idx, TD (&A)[RG][EPL], TD (&B)[NB][EPL]) {
         const int q = n0 - 1 + idx / SPB;
         const int cc = (idx % SPB) * 4 * EPL + EPL * lg;
-        const TD* Dq = q < n0 ? Drm + (size_t)leaf * BL * BL : (const TD*)nearB[q].d;
+        const TD* Dq = q < n0 ? Drm + (size_t)leaf * BL * BL : in_global<TD>(nearB[q].d);
         const int cl = q < n0 ? leaf : nearB[q].colLeaf;
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg) vload(Dq + (row0 + 16 * rg + lc) * BL + cc, A[rg]);
@@ -899,7 +900,7 @@ __device__ inline void near_otf(int leaf, int w, int row0, const float4* __restr
 // first instead, its sum multiplied by hiMul = 2^(E - Ea) into the FP16
 // group's units.
 template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false, int RG = BL / 16>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 2 : 1))) k_mf_phase2g(int S, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
                                                     const int32_t* __restrict__ gptrA,
                                                     const MfEntry* __restrict__ gentA, const TA* __restrict__ ZA,
                                                     const int32_t* __restrict__ ptrB, const MfEntry* __restrict__ entB,
@@ -921,7 +922,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
                       sizeof(typename Mfma<TD>::acc_t) == sizeof(typename MA::acc_t),
                   "one accumulator type per launch");
     constexpr int WPL = BL / 16 / RG;  // waves per leaf, RG 16-row groups each
-    const int blk = xcd_local(blockIdx.x, gridDim.x);
+    const int blk = xcd_chunked(blockIdx.x, chunk);
     // wave-uniform leaf (readfirstlane): scalar entry loads, no exec masks on
     // the entry loops.  FP64 phase 2 39.2 -> 38.1 ms at N = 2^20, 64
     // right-hand sides; the mixed kernel is slower that way (9.7 -> 10.2 ms,
@@ -1113,8 +1114,9 @@ __global__ void __launch_bounds__(256) k_colstats(int64_t ncols, const ColDesc* 
     const int lane = threadIdx.x & 63;
     const ColDesc d = cols[c];
     double su = 0, sv = 0, mu = 0, mv = 0;
+    const double *du = in_global<double>(d.u), *dv = in_global<double>(d.v);
     for (int i = lane; i < d.m; i += 64) {
-        const double u = d.u[i], v = d.v[i];
+        const double u = du[i], v = dv[i];
         su += u * u;
         sv += v * v;
         mu = fmax(mu, fabs(u));
@@ -1149,7 +1151,7 @@ __global__ void __launch_bounds__(256) k_cvt_cols(int64_t n, const CvCol* __rest
     const CvCol d = cols[c];
     const double inv = 1.0 / (double)d.scale;
     for (int i = lane; i < d.m; i += 64) {
-        const T v = d.src ? (T)(d.src[i] * inv) : (T)0;
+        const T v = d.src ? (T)(in_global<double>(d.src)[i] * inv) : (T)0;
         V[d.dst + urm_index<T>(d.col, i, d.m)] = v;
     }
 }
@@ -1164,7 +1166,7 @@ __global__ void __launch_bounds__(256) k_cvt_cols_split(int64_t n, const CvCol* 
     const CvCol d = cols[c];
     const double inv = 1.0 / (double)d.scale;
     for (int i = lane; i < d.m; i += 64) {
-        const double x = d.src ? d.src[i] * inv : 0.0;
+        const double x = d.src ? in_global<double>(d.src)[i] * inv : 0.0;
         const _Float16 hi = (_Float16)x;
         const size_t o = (size_t)d.dst + urm_index<_Float16>(d.col, i, d.m);
         V[o] = hi;
@@ -1190,7 +1192,7 @@ __global__ void __launch_bounds__(256) k_cvt_rowmajor(int64_t n, const TrTile* _
         double v = 0.0;
         if (c < t.cnt && r < t.m) {
             const CvCol d = cols[t.colDesc + c];
-            v = d.src ? d.src[r] / (double)d.scale : 0.0;
+            v = d.src ? in_global<double>(d.src)[r] / (double)d.scale : 0.0;
         }
         sh[cc][tx] = v;
     }
@@ -1213,7 +1215,7 @@ __global__ void __launch_bounds__(256) k_cvt_rowmajor_split(int64_t n, const TrT
         double v = 0.0;
         if (c < t.cnt && r < t.m) {
             const CvCol d = cols[t.colDesc + c];
-            v = d.src ? d.src[r] / (double)d.scale : 0.0;
+            v = d.src ? in_global<double>(d.src)[r] / (double)d.scale : 0.0;
         }
         sh[cc][tx] = v;
     }
@@ -1265,8 +1267,8 @@ __global__ void __launch_bounds__(256) k_near_blocks(int64_t n, const NearPair* 
         for (int j = 0; j < RG; ++j) acc[i][j] = v4d{0, 0, 0, 0};
     for (int a0 = 0; a0 < t.r; a0 += 4) {
         const bool ok = a0 + lg < t.r;
-        const double* A = t.A + (size_t)(a0 + lg) * BL + lc;
-        const double* B = t.B + (size_t)(a0 + lg) * BL + lc;
+        const double* A = in_global<double>(t.A) + (size_t)(a0 + lg) * BL + lc;
+        const double* B = in_global<double>(t.B) + (size_t)(a0 + lg) * BL + lc;
         double x[RG], y[RG];
 #pragma unroll
         for (int i = 0; i < RG; ++i) {
@@ -1910,6 +1912,20 @@ int phase1_chunk() {
 bool split_items(const MfGroup& G) { return G.numItems < 4096; }
 bool split_leaves(int S) { return S < 1024; }
 
+// Workgroups of phase 2 (x) for so many waves, and workgroups per XCD chunk
+// (y).  Passes of 16 right-hand sides: chunks of 8 are dealt to the XCDs in
+// turn, as one range of leaves per XCD does not balance where leaves differ in
+// cost (48 clouds in 2D and 3D, 8 right-hand sides, 3140 us a call with ranges,
+// 2740 with chunks of 8, 2700 of 4, 2760 of 16; N = 60000 3D 1025 -> 984, 120000
+// 2400 -> 2314).  Wider passes read more of z and X, which neighbours share in
+// an L2, and keep the ranges (64 right-hand sides at N = 100000 3D 5470 us, with
+// chunks 5515).
+int2 phase2_grid(int waves, bool narrow) {
+    const int wgs = (waves + 3) / 4, range = (wgs + 7) / 8;
+    const int chunk = std::max(1, narrow ? std::min(kP2Chunk, range) : range);
+    return make_int2((wgs + 8 * chunk - 1) / (8 * chunk) * (8 * chunk), chunk);
+}
+
 template <class T, int CG, int NB>
 void phase1(Context& c, MfGroup& G, const T* Xb, int sh, int kvalid, int xcdChunk = -1) {
     if (G.numItems == 0) return;
@@ -1990,6 +2006,7 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
         const int* gp = G.grouped ? G.grpPtr.p : nullptr;
         const MfEntry* ge = G.grouped ? G.grpEntries.p : nullptr;
         const bool split = split_leaves(P.S);
+        const int2 pg = phase2_grid(P.S * (split ? P.b / 16 : 1), NB == 1);
         auto pick = [&](auto b, auto ucm) {
             constexpr int B = decltype(b)::value;
             constexpr bool U = decltype(ucm)::value;
@@ -2000,7 +2017,7 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
         using B32 = std::integral_constant<int, 32>;
         auto k2 = P.b == 64 ? (P.ucm ? pick(B64{}, std::true_type{}) : pick(B64{}, std::false_type{}))
                             : (P.ucm ? pick(B32{}, std::true_type{}) : pick(B32{}, std::false_type{}));
-        k2<<<(P.S * (split ? P.b / 16 : 1) + 3) / 4, 256, 0, c.stream>>>(P.S, G.leafPtr.p, G.entries.p, gp, ge, (const double*)G.zt.p,
+        k2<<<pg.x, 256, 0, c.stream>>>(P.S, pg.y, G.leafPtr.p, G.entries.p, gp, ge, (const double*)G.zt.p,
                                                 nullptr, nullptr, nullptr, nullptr, nullptr, (const double*)P.Drm.p,
                                                 P.nearPtr.p, P.near.p, Xb, Yo, ldo, kk, nullptr, 1.f, nullptr, nullptr,
                                                 0.f, nullptr, nullptr, 0, 0, 1.f);
@@ -2052,9 +2069,10 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
         const bool spa = Ghi.split == 2;
         // a split group's z is FP16 hi + lo (the kernel's ZA), else FP32
         const bool split = !spa && split_leaves(P.S);
+        const int2 pg = phase2_grid(P.S * (split ? P.b / 16 : 1), NB == 1);
         auto launch = [&](auto k2, const auto* za) {
-            k2<<<(P.S * (split ? P.b / 16 : 1) + 3) / 4, 256, 0, c.stream>>>(
-                P.S, Ghi.leafPtr.p, Ghi.entries.p, gr ? Ghi.grpPtr.p : nullptr, gr ? Ghi.grpEntries.p : nullptr, za,
+            k2<<<pg.x, 256, 0, c.stream>>>(
+                P.S, pg.y, Ghi.leafPtr.p, Ghi.entries.p, gr ? Ghi.grpPtr.p : nullptr, gr ? Ghi.grpEntries.p : nullptr, za,
                 Glo.leafPtr.p, Glo.entries.p, gr ? Glo.grpPtr.p : nullptr, gr ? Glo.grpEntries.p : nullptr,
                 (const _Float16*)Glo.zt.p, (const float*)P.Drm.p, P.nearOtf ? P.gnearPtr.p : P.nearPtr.p,
                 P.nearOtf ? P.gnear.p : P.near.p, Xb, Yo, ldo, kk, P.xscale.p, P.loMul,

@@ -171,6 +171,19 @@ __device__ inline size_t xb_index(int64_t row, int s, int sh) {
 constexpr int kPipe = 4;   // phase 2
 constexpr int kPipe1 = 2;  // phase 1
 constexpr int kP2Chunk = 8;  // phase2_grid
+// 16 right-hand sides, phase 2: whether the ring of steps runs without a branch
+// round its loads (lr_rows, dense_rows).  With branches the compiler merges
+// what may be in flight on either way and waits for all of it; without, each
+// step waits for its own operands, and the steps past a list's end are loaded
+// and multiplied by zero.  Calls of 16 with branches -> without: mixed N = 4096
+// 2D 53 -> 48 us, 16384 74 -> 65, 65536 147 -> 135; 16384 3D 131 -> 114,
+// 120000 3D 798 -> 745; FP64 4096 2D 59 -> 57, 16384 3D 236 -> 222, 60000 3D
+// 1020 -> 980.  FP64 with 32-row leaves in one wave is the exception (65536 2D
+// 256 -> 273, 48 clouds 2690 -> 2750): short lists, read at memory speed.
+template <class T>
+constexpr bool in_line(int rg) {
+    return sizeof(T) < 8 || rg != 2;
+}
 
 // ---- phase 1 ---------------------------------------------------------------
 // SPLIT (T = FP16): the FP32 group of a mixed plan with V held as FP16 hi +
@@ -563,6 +576,92 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
             for (int nb = 0; nb < NB; ++nb) vzero(B[nb]);
         }
     };
+    if constexpr (NB == 1 && in_line<T>(RG)) {
+        // kPipe steps of the list in flight, the next entry's descriptor read
+        // an entry ahead.  No branch goes round a load: past the end the last
+        // entry's are repeated, a lane past the rank or a right-hand side past
+        // kvalid reads a neighbour's (and is cleared, or never stored), so that
+        // a wait names the step it needs and not all that is in flight.
+        constexpr int P = RG * sizeof(T) >= 32 ? 3 : kPipe;
+        T pa[P][RG][VL], pb[P][VL];
+        int left[P], ranks[P];  // columns from the step's first on: padded, present
+        int e = e0, c0 = 0;
+        const MfEntry* pe = ents + e;
+        const void* eu = pe->u;
+        int erpad = pe->rpad, ezcol = pe->zcol, erank = pe->rank, eld = pe->ld;
+        pe = ents + min(e + 1, e1 - 1);
+        const void* nu = pe->u;
+        int nrpad = pe->rpad, nzcol = pe->zcol, nrank = pe->rank, nld = pe->ld;
+        const int sv = lc < kvalid ? lc : 0;
+        auto fill = [&](int d) {
+            const int w = erpad - c0;
+            left[d] = e < e1 ? w : 0;
+            ranks[d] = erank - c0;
+            const int lq = VL * lg < w ? lg : 0;
+            const int pstride = 16 * E16 * (min(SS, w) / VL);
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) {
+                if (UCM) {
+                    const T* U = in_global<T>(eu) + rowOff + 16 * rg + lc;
+#pragma unroll
+                    for (int q = 0; q < VL; ++q)
+                        pa[d][rg][q] = __builtin_nontemporal_load(U + (size_t)min(c0 + VL * lq + q, erank - 1) * eld);
+                } else {
+                    const T* U = in_global<T>(eu) + (size_t)(rowOff / 16 + rg) * 16 * erpad + (size_t)16 * c0;
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) vload16_nt(U + (16 * lq + lc) * E16 + p * pstride, &pa[d][rg][p * E16]);
+                }
+            }
+            constexpr int ZP = z_piece<T>();
+            const T* zp = Z + zt_index<T, NR>(ezcol + c0 + VL * lq, sv);
+            if constexpr (ZP == E16) {
+#pragma unroll
+                for (int p = 0; p < VL / ZP; ++p) vload16(zp + p * NR * ZP, &pb[d][p * ZP]);
+            } else {
+                vload(zp, pb[d]);
+            }
+            c0 += SS;
+            const bool nxt = c0 >= erpad;
+            e += nxt ? 1 : 0;
+            c0 = nxt ? 0 : c0;
+            eu = nxt ? nu : eu;
+            erpad = nxt ? nrpad : erpad;
+            ezcol = nxt ? nzcol : ezcol;
+            erank = nxt ? nrank : erank;
+            eld = nxt ? nld : eld;
+            pe = ents + min(e + 1, e1 - 1);
+            nu = pe->u;
+            nrpad = pe->rpad;
+            nzcol = pe->zcol;
+            nrank = pe->rank;
+            nld = pe->ld;
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay in the order of the steps
+        };
+#pragma unroll
+        for (int d = 0; d < P; ++d) fill(d);
+        while (left[0] > 0) {  // a round: its steps past the end multiply zeros
+#pragma unroll
+            for (int d = 0; d < P; ++d) {
+                if (min(left[d], UCM ? ranks[d] : left[d]) < SS) {
+                    const bool in = VL * lg < left[d];
+#pragma unroll
+                    for (int q = 0; q < VL; ++q) {
+                        const bool inA = UCM ? VL * lg + q < ranks[d] : in;
+#pragma unroll
+                        for (int rg = 0; rg < RG; ++rg) pa[d][rg][q] = inA ? pa[d][rg][q] : (T)0;
+                        pb[d][q] = in ? pb[d][q] : (T)0;
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < VL / MX::KL; ++q)
+#pragma unroll
+                    for (int rg = 0; rg < RG; ++rg)
+                        acc[rg][0] = MX::op(MX::make(&pa[d][rg][q * MX::KL]), MX::make(&pb[d][q * MX::KL]), acc[rg][0]);
+                fill(d);
+            }
+        }
+        return;
+    }
     if constexpr (NB == 1) {
         // kPipe steps of the list in flight; the next entry's descriptor is
         // read an entry ahead
@@ -754,6 +853,56 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
             }
         }
     };
+    if constexpr (NB == 1 && in_line<TD>(RG)) {
+        // a ring as in lr_rows; the next block's descriptor is read a block ahead
+        constexpr int P = RG * sizeof(TD) >= 32 ? 2 : (SPB < kPipe ? SPB : kPipe);
+        TD pa[P][RG][EPL], pb[P][EPL];
+        const int sv = lc < kvalid ? lc : 0;
+        int q = n0, c0 = 0, cl = leaf;
+        const TD* Dq = Drm + (size_t)leaf * BL * BL;
+        const TD* nD = Dq;
+        int ncl = leaf;
+        if (n0 < n1) {
+            nD = in_global<TD>(nearB[n0].d);
+            ncl = nearB[n0].colLeaf;
+        }
+        auto fill = [&](int d) {
+            const int cc = c0 + EPL * lg;
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) vload(Dq + (row0 + 16 * rg + lc) * BL + cc, pa[d][rg]);
+            if constexpr (sizeof(TD) < 8) {
+#pragma unroll
+                for (int p = 0; p < EPL / 4; ++p)
+                    vload16(Xb + xb_index<NR>((int64_t)cl * BL + cc + 4 * p, sv, 2), &pb[d][4 * p]);
+            } else {
+                vload(Xb + ((size_t)cl * NR + sv) * BL + cc, pb[d]);
+            }
+            c0 += 4 * EPL;
+            if (c0 == BL) {
+                c0 = 0;
+                Dq = nD;
+                cl = ncl;
+                if (++q < n1) {
+                    nD = in_global<TD>(nearB[q].d);
+                    ncl = nearB[q].colLeaf;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int d = 0; d < P; ++d) fill(d);
+        for (int i0 = 0; i0 < total; i0 += P)
+#pragma unroll
+            for (int d = 0; d < P; ++d) {
+                if (i0 + d < total)
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e)
+#pragma unroll
+                        for (int rg = 0; rg < RG; ++rg) acc[rg][0] = MD::op(pa[d][rg][e], pb[d][e], acc[rg][0]);
+                fill(d);
+            }
+        return;
+    }
     if constexpr (NB == 1) {
         TD pa[kPipe][RG][EPL], pb[kPipe][NB][EPL];
 #pragma unroll
@@ -900,7 +1049,7 @@ __device__ inline void near_otf(int leaf, int w, int row0, const float4* __restr
 // first instead, its sum multiplied by hiMul = 2^(E - Ea) into the FP16
 // group's units.
 template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false, int RG = BL / 16>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA || (NB == 1 && in_line<TA>(RG)) ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
                                                     const int32_t* __restrict__ gptrA,
                                                     const MfEntry* __restrict__ gentA, const TA* __restrict__ ZA,
                                                     const int32_t* __restrict__ ptrB, const MfEntry* __restrict__ entB,
@@ -927,7 +1076,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ? 
     // the entry loops.  FP64 phase 2 39.2 -> 38.1 ms at N = 2^20, 64
     // right-hand sides; the mixed kernel is slower that way (9.7 -> 10.2 ms,
     // measured) and keeps the per-lane index.
-    const int w = sizeof(TA) == 8 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
+    const int w = sizeof(TA) == 8 || NB == 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, lg = lane >> 4, lc = lane & 15;
     const int unit = 4 * blk + w, leaf = unit / WPL, row0 = WPL > 1 ? 16 * RG * (unit % WPL) : 0;
     const int grp = leaf >> 2, wl = leaf & 3;

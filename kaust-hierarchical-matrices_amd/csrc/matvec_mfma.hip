@@ -171,18 +171,21 @@ __device__ inline size_t xb_index(int64_t row, int s, int sh) {
 constexpr int kPipe = 4;   // phase 2
 constexpr int kPipe1 = 2;  // phase 1
 constexpr int kP2Chunk = 8;  // phase2_grid
-// 16 right-hand sides, phase 2: whether the ring of steps runs without a branch
-// round its loads (lr_rows, dense_rows).  With branches the compiler merges
-// what may be in flight on either way and waits for all of it; without, each
-// step waits for its own operands, and the steps past a list's end are loaded
-// and multiplied by zero.  Calls of 16 with branches -> without: mixed N = 4096
-// 2D 53 -> 48 us, 16384 74 -> 65, 65536 147 -> 135; 16384 3D 131 -> 114,
-// 120000 3D 798 -> 745; FP64 4096 2D 59 -> 57, 16384 3D 236 -> 222, 60000 3D
-// 1020 -> 980.  FP64 with 32-row leaves in one wave is the exception (65536 2D
-// 256 -> 273, 48 clouds 2690 -> 2750): short lists, read at memory speed.
-template <class T>
+// Phase 2: whether the ring of steps runs without a branch round its loads
+// (lr_rows, dense_rows).  With branches the compiler merges what may be in
+// flight on either way and waits for all of it; without, each step waits for
+// its own operands, and the steps past a list's end are loaded and multiplied
+// by zero.  Calls with branches -> without, 16 right-hand sides mixed: N = 4096
+// 2D 53 -> 48 us, 65536 147 -> 135, 16384 3D 131 -> 114, 120000 3D 798 -> 745;
+// FP64 4096 2D 59 -> 57, 16384 3D 236 -> 222, 60000 3D 1020 -> 980.  64 (two
+// steps in flight; before, one and copies between two buffers): FP64 N = 60000
+// 3D 2460 -> 2010, 100000 5460 -> 4690, 65536 2D 590 -> 561; mixed 60000 3D
+// 556 -> 512, 65536 2D 220 -> 205.  FP64, 16 right-hand sides, 32-row leaves in
+// one wave is the exception (65536 2D 256 -> 273, 48 clouds 2690 -> 2750):
+// short lists, read at memory speed.
+template <class T, int NB>
 constexpr bool in_line(int rg) {
-    return sizeof(T) < 8 || rg != 2;
+    return NB > 1 || sizeof(T) < 8 || rg != 2;
 }
 
 // ---- phase 1 ---------------------------------------------------------------
@@ -532,7 +535,6 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
     using MX = typename std::conditional<std::is_same<T, _Float16>::value, Mfma32h, M>::type;  // as in phase 1
     constexpr int KL = M::KL, VL = 4 * KL, SS = 16 * KL, NR = 16 * NB, E16 = 16 / (int)sizeof(T), NP = VL / E16;
     if (e0 >= e1) return;
-    T a[RG][VL], bz[NB][VL], an[RG][VL], bn[NB][VL];
     auto load = [&](const MfEntry& en, int c0, T (&A)[RG][VL], T (&B)[NB][VL]) {
         const int cc = c0 + VL * lg;
         if (cc < en.rpad) {
@@ -576,14 +578,14 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
             for (int nb = 0; nb < NB; ++nb) vzero(B[nb]);
         }
     };
-    if constexpr (NB == 1 && in_line<T>(RG)) {
+    if constexpr (in_line<T, NB>(RG)) {
         // kPipe steps of the list in flight, the next entry's descriptor read
         // an entry ahead.  No branch goes round a load: past the end the last
         // entry's are repeated, a lane past the rank or a right-hand side past
         // kvalid reads a neighbour's (and is cleared, or never stored), so that
         // a wait names the step it needs and not all that is in flight.
-        constexpr int P = RG * sizeof(T) >= 32 ? 3 : kPipe;
-        T pa[P][RG][VL], pb[P][VL];
+        constexpr int P = NB > 1 ? 2 : (RG * sizeof(T) >= 32 ? 3 : kPipe);
+        T pa[P][RG][VL], pb[P][NB][VL];
         int left[P], ranks[P];  // columns from the step's first on: padded, present
         int e = e0, c0 = 0;
         const MfEntry* pe = ents + e;
@@ -592,7 +594,6 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
         pe = ents + min(e + 1, e1 - 1);
         const void* nu = pe->u;
         int nrpad = pe->rpad, nzcol = pe->zcol, nrank = pe->rank, nld = pe->ld;
-        const int sv = lc < kvalid ? lc : 0;
         auto fill = [&](int d) {
             const int w = erpad - c0;
             left[d] = e < e1 ? w : 0;
@@ -613,12 +614,15 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
                 }
             }
             constexpr int ZP = z_piece<T>();
-            const T* zp = Z + zt_index<T, NR>(ezcol + c0 + VL * lq, sv);
-            if constexpr (ZP == E16) {
 #pragma unroll
-                for (int p = 0; p < VL / ZP; ++p) vload16(zp + p * NR * ZP, &pb[d][p * ZP]);
-            } else {
-                vload(zp, pb[d]);
+            for (int nb = 0; nb < NB; ++nb) {
+                const T* zp = Z + zt_index<T, NR>(ezcol + c0 + VL * lq, 16 * nb + lc < kvalid ? 16 * nb + lc : 0);
+                if constexpr (ZP == E16) {
+#pragma unroll
+                    for (int p = 0; p < VL / ZP; ++p) vload16(zp + p * NR * ZP, &pb[d][nb][p * ZP]);
+                } else {
+                    vload(zp, pb[d][nb]);
+                }
             }
             c0 += SS;
             const bool nxt = c0 >= erpad;
@@ -649,14 +653,17 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
                         const bool inA = UCM ? VL * lg + q < ranks[d] : in;
 #pragma unroll
                         for (int rg = 0; rg < RG; ++rg) pa[d][rg][q] = inA ? pa[d][rg][q] : (T)0;
-                        pb[d][q] = in ? pb[d][q] : (T)0;
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb) pb[d][nb][q] = in ? pb[d][nb][q] : (T)0;
                     }
                 }
 #pragma unroll
                 for (int q = 0; q < VL / MX::KL; ++q)
 #pragma unroll
                     for (int rg = 0; rg < RG; ++rg)
-                        acc[rg][0] = MX::op(MX::make(&pa[d][rg][q * MX::KL]), MX::make(&pb[d][q * MX::KL]), acc[rg][0]);
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[rg][nb] = MX::op(MX::make(&pa[d][rg][q * MX::KL]), MX::make(&pb[d][nb][q * MX::KL]), acc[rg][nb]);
                 fill(d);
             }
         }
@@ -695,40 +702,6 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
                             acc[rg][0] = MX::op(MX::make(&pa[d][rg][q * MX::KL]), MX::make(&pb[d][0][q * MX::KL]), acc[rg][0]);
                     fill(d);
                 }
-        return;
-    }
-    int e = e0, c0 = 0;
-    MfEntry en = ents[e];
-    load(en, 0, a, bz);
-    while (true) {
-        int ne = e, nc = c0 + SS;
-        MfEntry nen = en;
-        if (nc >= en.rpad) {
-            ne = e + 1;
-            nc = 0;
-            if (ne < e1) nen = ents[ne];
-        }
-        const bool more = ne < e1;
-        if (more) load(nen, nc, an, bn);
-#pragma unroll
-        for (int q = 0; q < VL / MX::KL; ++q)
-#pragma unroll
-            for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    acc[rg][nb] = MX::op(MX::make(&a[rg][q * MX::KL]), MX::make(&bz[nb][q * MX::KL]), acc[rg][nb]);
-        if (!more) break;
-#pragma unroll
-        for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-            for (int q = 0; q < VL; ++q) a[rg][q] = an[rg][q];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int q = 0; q < VL; ++q) bz[nb][q] = bn[nb][q];
-        e = ne;
-        c0 = nc;
-        en = nen;
     }
 }
 
@@ -830,7 +803,6 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
     static_assert(SPB >= 1, "a step spans at most one block row");
     const int n0 = nearPtr ? nearPtr[leaf] : 0, n1 = nearPtr ? nearPtr[leaf + 1] : 0;
     const int total = (n1 - n0 + 1) * SPB;
-    TD a[RG][EPL], bx[NB][EPL], an[RG][EPL], bn[NB][EPL];
     auto dload = [&](int idx, TD (&A)[RG][EPL], TD (&B)[NB][EPL]) {
         const int q = n0 - 1 + idx / SPB;
         const int cc = (idx % SPB) * 4 * EPL + EPL * lg;
@@ -853,11 +825,10 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
             }
         }
     };
-    if constexpr (NB == 1 && in_line<TD>(RG)) {
+    if constexpr (in_line<TD, NB>(RG)) {
         // a ring as in lr_rows; the next block's descriptor is read a block ahead
         constexpr int P = RG * sizeof(TD) >= 32 ? 2 : (SPB < kPipe ? SPB : kPipe);
-        TD pa[P][RG][EPL], pb[P][EPL];
-        const int sv = lc < kvalid ? lc : 0;
+        TD pa[P][RG][EPL], pb[P][NB][EPL];
         int q = n0, c0 = 0, cl = leaf;
         const TD* Dq = Drm + (size_t)leaf * BL * BL;
         const TD* nD = Dq;
@@ -870,12 +841,16 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
             const int cc = c0 + EPL * lg;
 #pragma unroll
             for (int rg = 0; rg < RG; ++rg) vload(Dq + (row0 + 16 * rg + lc) * BL + cc, pa[d][rg]);
-            if constexpr (sizeof(TD) < 8) {
 #pragma unroll
-                for (int p = 0; p < EPL / 4; ++p)
-                    vload16(Xb + xb_index<NR>((int64_t)cl * BL + cc + 4 * p, sv, 2), &pb[d][4 * p]);
-            } else {
-                vload(Xb + ((size_t)cl * NR + sv) * BL + cc, pb[d]);
+            for (int nb = 0; nb < NB; ++nb) {
+                const int sv = 16 * nb + lc < kvalid ? 16 * nb + lc : 0;
+                if constexpr (sizeof(TD) < 8) {  // FP32 right-hand sides in blocks of 4 rows
+#pragma unroll
+                    for (int p = 0; p < EPL / 4; ++p)
+                        vload16(Xb + xb_index<NR>((int64_t)cl * BL + cc + 4 * p, sv, 2), &pb[d][nb][4 * p]);
+                } else {  // FP64: blocks of one leaf
+                    vload(Xb + ((size_t)cl * NR + sv) * BL + cc, pb[d][nb]);
+                }
             }
             c0 += 4 * EPL;
             if (c0 == BL) {
@@ -894,11 +869,14 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
         for (int i0 = 0; i0 < total; i0 += P)
 #pragma unroll
             for (int d = 0; d < P; ++d) {
-                if (i0 + d < total)
+                if (SPB % P == 0 || i0 + d < total)
 #pragma unroll
                     for (int e = 0; e < EPL; ++e)
 #pragma unroll
-                        for (int rg = 0; rg < RG; ++rg) acc[rg][0] = MD::op(pa[d][rg][e], pb[d][e], acc[rg][0]);
+                        for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+                            for (int nb = 0; nb < NB; ++nb)
+                                acc[rg][nb] = MD::op(pa[d][rg][e], pb[d][nb][e], acc[rg][nb]);
                 fill(d);
             }
         return;
@@ -918,28 +896,6 @@ __device__ inline void dense_rows(int leaf, int row0, const TD* __restrict__ Drm
                         for (int rg = 0; rg < RG; ++rg) acc[rg][0] = MD::op(pa[d][rg][e], pb[d][0][e], acc[rg][0]);
                     if (i0 + d + kPipe < total) dload(i0 + d + kPipe, pa[d], pb[d]);
                 }
-        return;
-    }
-    dload(0, a, bx);
-    for (int idx = 0; idx < total; ++idx) {
-        const bool more = idx + 1 < total;
-        if (more) dload(idx + 1, an, bn);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e)
-#pragma unroll
-            for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) acc[rg][nb] = MD::op(a[rg][e], bx[nb][e], acc[rg][nb]);
-        if (more) {
-#pragma unroll
-            for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) a[rg][e] = an[rg][e];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) bx[nb][e] = bn[nb][e];
-        }
     }
 }
 
@@ -1049,7 +1005,7 @@ __device__ inline void near_otf(int leaf, int w, int row0, const float4* __restr
 // first instead, its sum multiplied by hiMul = 2^(E - Ea) into the FP16
 // group's units.
 template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false, int RG = BL / 16>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA || (NB == 1 && in_line<TA>(RG)) ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA || (NB == 1 && in_line<TA, NB>(RG)) ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
                                                     const int32_t* __restrict__ gptrA,
                                                     const MfEntry* __restrict__ gentA, const TA* __restrict__ ZA,
                                                     const int32_t* __restrict__ ptrB, const MfEntry* __restrict__ entB,
@@ -1072,11 +1028,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA ||
                   "one accumulator type per launch");
     constexpr int WPL = BL / 16 / RG;  // waves per leaf, RG 16-row groups each
     const int blk = xcd_chunked(blockIdx.x, chunk);
-    // wave-uniform leaf (readfirstlane): scalar entry loads, no exec masks on
-    // the entry loops.  FP64 phase 2 39.2 -> 38.1 ms at N = 2^20, 64
-    // right-hand sides; the mixed kernel is slower that way (9.7 -> 10.2 ms,
-    // measured) and keeps the per-lane index.
-    const int w = sizeof(TA) == 8 || NB == 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)(threadIdx.x >> 6);
+    // wave-uniform leaf (readfirstlane): the entries are scalar loads, which
+    // leave the count of the operand loads in flight alone
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63, lg = lane >> 4, lc = lane & 15;
     const int unit = 4 * blk + w, leaf = unit / WPL, row0 = WPL > 1 ? 16 * RG * (unit % WPL) : 0;
     const int grp = leaf >> 2, wl = leaf & 3;

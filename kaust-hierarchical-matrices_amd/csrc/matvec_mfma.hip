@@ -222,11 +222,9 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     // The item index is the same in every lane of the wave.  Declared so
     // (readfirstlane), the item loads into scalar registers and the loop runs
     // without exec masks: FP32/FP16 phase 1 8.3 -> 8.0 ms at N = 2^20, 64
-    // right-hand sides; FP64 with 16 (256-cloud batch) 19.15 -> 18.95 ms per
-    // call.  The FP64 kernels with 48 and 64 are scheduled worse that way (64:
-    // 36.4 -> 40.7 ms, measured) and keep the per-lane index.
+    // right-hand sides.
     const int wv = wg * 4 + (int)(threadIdx.x >> 6);
-    const int unit = (sizeof(T) < 8 || NB <= 2) ? __builtin_amdgcn_readfirstlane(wv) : wv;
+    const int unit = __builtin_amdgcn_readfirstlane(wv);
     constexpr int UPI = kMfCols / 16 / CG;  // waves per item, CG 16-column groups each
     const int wid = unit / UPI, g0 = UPI > 1 ? (unit % UPI) * CG : 0;
     if (wid >= nItems) return;
@@ -240,43 +238,22 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
     for (int g = 0; g < CG; ++g)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[g][nb] = typename M::accv{0, 0, 0, 0};
-    // FP64 with 48 or 64 right-hand sides and FP16: software pipelined, the
+    // FP64: kPipe1 steps in flight without a branch round a load (in_line; 64
+    // right-hand sides, before with one step ahead, branches and copies: whole
+    // call at N = 60000 3D 2005 -> 1815 us, 100000 4640 -> 4080, 65536 2D 562
+    // -> 485; 32 at 100000 2797 -> 2700; 16 at 4096 2D 56 -> 48).  FP16: the
     // operands of super-step r0 + 16*KL are in flight while the MFMAs of
-    // super-step r0 run (FP64 36.4 ms vs 39.1 without, at N = 2^20; FP16
-    // 4.4 -> 4.2 ms with the fragment-ordered copies).  FP64 with 16 or
-    // 32 and FP32: no register double buffer -- the registers it frees buy
-    // more waves per SIMD, which hide the load latency better (FP64 16 RHS
-    // 16.6 -> 15.9 ms; 32 RHS at N = 60000 3D, whole call 1621 -> 1529 us;
-    // FP32 slower with it).
-    constexpr bool DEEP = sizeof(T) == 8 && NB == 1;
-    constexpr bool PF = !DEEP && !SPLIT && ((sizeof(T) == 8 && NB > 2) || sizeof(T) == 2);
+    // super-step r0 run (4.4 -> 4.2 ms at N = 2^20 with the fragment-ordered
+    // copies).  FP32: no register double buffer -- the registers it frees buy
+    // more waves per SIMD, which hide the load latency better.
+    constexpr bool DEEP = sizeof(T) == 8;
+    constexpr bool PF = !SPLIT && sizeof(T) == 2;
     T a[CG][VL], bx[NB][VL], an[CG][VL], bn[NB][VL];
     constexpr int E16 = 16 / (int)sizeof(T), NP = VL / E16;
     auto load = [&](int r0, T (&A)[CG][VL], T (&B)[NB][VL]) {
         const int rr = r0 + VL * lg;
         const bool rok = rr < it.rows;
-        if constexpr (sizeof(T) == 8 && VF) {
-            // FP64 copies in fragment order: whole cache lines per load
-            // instruction for V; the right-hand sides in blocks of a leaf
-            const int pstride = 16 * E16 * (min(16 * KL, it.rows - r0) / VL);
-#pragma unroll
-            for (int g = 0; g < CG; ++g) {
-                if (rok && 16 * (g0 + g) + lc < it.ncols) {
-                    const T* vp = V + (size_t)(g0 + g) * 16 * it.ld + (size_t)16 * r0 + (16 * lg + lc) * E16;
-#pragma unroll
-                    for (int p = 0; p < NP; ++p) vload16_nt(vp + p * pstride, &A[g][p * E16]);
-                } else {
-                    vzero(A[g]);
-                }
-            }
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                if (rok && 16 * nb + lc < kvalid)
-                    vload(Xb + xb_index<NR>((int64_t)it.xoff + rr, 16 * nb + lc, sh), B[nb]);
-                else
-                    vzero(B[nb]);
-            }
-        } else if constexpr (sizeof(T) < 8) {
+        if constexpr (sizeof(T) < 8) {
             // FP32/FP16 copies in fragment order (V column c, row r at
             // urm_index(c, r, m) of its run; the item points at its first
             // column block and row chunk), the right-hand sides in blocks
@@ -302,21 +279,6 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
                 } else {
                     vzero(B[nb]);
                 }
-            }
-        } else {
-#pragma unroll
-            for (int g = 0; g < CG; ++g) {
-                const int col = 16 * (g0 + g) + lc;
-                if (rok && col < it.ncols) vload_f(V + (size_t)col * it.ld + rr, A[g]);
-                else vzero(A[g]);
-            }
-            // right-hand sides past kvalid are zero in Xb: not loaded
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                if (rok && 16 * nb + lc < kvalid)
-                    vload(Xb + xb_index<NR>((int64_t)it.xoff + rr, 16 * nb + lc, sh), B[nb]);
-                else
-                    vzero(B[nb]);
             }
         }
     };
@@ -348,24 +310,52 @@ __global__ void __launch_bounds__(256) k_mf_phase1(const MfItem* __restrict__ it
         }
     };
     if constexpr (DEEP) {
+        // kPipe1 steps of 16 rows in flight (an item's rows are a multiple of
+        // 32), no branch round a load (lr_rows below): columns past ncols and
+        // right-hand sides past kvalid read a neighbour's, their sums are not used
         constexpr int SS = 16 * KL;
         T pa[kPipe1][CG][VL], pb[kPipe1][NB][VL];
+        int col[CG];
 #pragma unroll
-        for (int d = 0; d < kPipe1; ++d)
-            if (d * SS < it.rows) load(d * SS, pa[d], pb[d]);
-        for (int r0 = 0; r0 < it.rows; r0 += kPipe1 * SS)
+        for (int g = 0; g < CG; ++g) col[g] = min(16 * (g0 + g) + lc, it.ncols - 1);
+        auto fill = [&](int d, int r0) {
+            const int rr = r0 + VL * lg;
 #pragma unroll
-            for (int d = 0; d < kPipe1; ++d) {
-                const int r = r0 + d * SS;
-                if (r < it.rows) {
+            for (int g = 0; g < CG; ++g) {
+                if constexpr (VF) {
+                    // FP64 copies in fragment order: whole cache lines per
+                    // load instruction for V
+                    const T* vp = V + (size_t)(col[g] >> 4) * 16 * it.ld + (size_t)16 * r0 + (16 * lg + (col[g] & 15)) * E16;
 #pragma unroll
-                    for (int e = 0; e < VL / MX::KL; ++e)
-#pragma unroll
-                        for (int g = 0; g < CG; ++g)
-                            acc[g][0] = MX::op(MX::make(&pa[d][g][e * MX::KL]), MX::make(&pb[d][0][e * MX::KL]), acc[g][0]);
-                    if (r + kPipe1 * SS < it.rows) load(r + kPipe1 * SS, pa[d], pb[d]);
+                    for (int p = 0; p < NP; ++p) vload16_nt(vp + p * 16 * E16 * (SS / VL), &pa[d][g][p * E16]);
+                } else {
+                    vload_f(V + (size_t)col[g] * it.ld + rr, pa[d][g]);
                 }
             }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                vload(Xb + xb_index<NR>((int64_t)it.xoff + rr, 16 * nb + lc < kvalid ? 16 * nb + lc : 0, sh), pb[d][nb]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto mult = [&](int d) {
+#pragma unroll
+            for (int e = 0; e < VL / MX::KL; ++e)
+#pragma unroll
+                for (int g = 0; g < CG; ++g)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+                        acc[g][nb] = MX::op(MX::make(&pa[d][g][e * MX::KL]), MX::make(&pb[d][nb][e * MX::KL]), acc[g][nb]);
+        };
+#pragma unroll
+        for (int d = 0; d < kPipe1; ++d) fill(d, d * SS);
+        for (int r0 = kPipe1 * SS; r0 < it.rows; r0 += kPipe1 * SS)
+#pragma unroll
+            for (int d = 0; d < kPipe1; ++d) {
+                mult(d);
+                fill(d, r0 + d * SS);
+            }
+#pragma unroll
+        for (int d = 0; d < kPipe1; ++d) mult(d);
     }
     if (PF) load(0, a, bx);
     for (int r0 = 0; !DEEP && r0 < it.rows; r0 += 16 * KL) {

@@ -136,7 +136,8 @@ hmx_status hmx_constructKDTreeBatch(hmx_context* ctx, int32_t count, const uint3
 hmx_status hmx_kdtree_info(const hmx_kdtree* tree, uint32_t* numSegments, uint32_t* segmentSize,
                            uint32_t* numLevels);
 /* host copies: perm[n] (segmentIndices), offsets[numSegments+1] (segmentOffsets),
-   bbmin/bbmax[(2^(numLevels+1)-1)*d] laid out [level][node][dim] (level l at node 2^l-1);
+   bbmin/bbmax[(2^(numLevels+1)-1)*d] laid out [level][node][dim] (level l at node 2^l-1),
+   zero where a level has no box (the leaves, absent POWER_OF_TWO_ON_LEFT segments);
    any pointer may be NULL */
 hmx_status hmx_kdtree_copy(hmx_context* ctx, const hmx_kdtree* tree, int32_t* perm, int32_t* offsets,
                            double* bbmin, double* bbmax);

@@ -54,10 +54,14 @@ struct KdSmall {
 };
 
 // ---- large segments ------------------------------------------------------------
-// points interleaved (x, y, z, 0), identity permutation, 64-bit sort keys
+// points interleaved (x, y, z, 0), identity permutation, and zeros in the box
+// slots (nbox values): no level fills those of the leaves and of segments a
+// tree does not have
 __global__ void __launch_bounds__(256) k_kd_init(int64_t n, uint32_t d, const double* __restrict__ p,
-                                                 double4* __restrict__ P4, int32_t* __restrict__ perm) {
+                                                 double4* __restrict__ P4, int32_t* __restrict__ perm, int64_t nbox,
+                                                 double* __restrict__ bbmin, double* __restrict__ bbmax) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < nbox) bbmin[e] = bbmax[e] = 0.0;
     if (e >= n) return;
     perm[e] = (int32_t)e;
     if (!P4) return;
@@ -673,7 +677,9 @@ static void kd_forest(Context& c, uint32_t d, std::vector<KdJob>& jobs) {
 
     DBuf<double4> P4;
     if (large) P4.alloc((size_t)ntot);
-    k_kd_init<<<(unsigned)((ntot + 255) / 256), 256, 0, c.stream>>>(ntot, d, P, P4.p, perm);
+    const int64_t nbox = nodes * d;
+    k_kd_init<<<(unsigned)((std::max(ntot, nbox) + 255) / 256), 256, 0, c.stream>>>(ntot, d, P, P4.p, perm, nbox,
+                                                                                    bbminF->p, bbmaxF->p);
     HMX_LAUNCHED();
     if (large) {
         int mostSegs = pre.nseg, mostChunks = pre.nchunk;

@@ -238,10 +238,9 @@ void hmatvec_grad_factors(Context& c, HMatrix& h, uint32_t k, const double* X, c
     const bool gather = P.npad != (int64_t)h.n;
     const bool copy = !gather && (((uintptr_t)X | (uintptr_t)dY) & 15);
     const int NB = mf_pass_blocks(k), NR = 16 * NB;
-    if ((gather || copy) && P.wsK < (uint32_t)NR) {
-        P.Xp.alloc((size_t)P.npad * NR);
-        P.Wp.alloc((size_t)P.npad * NR);
-        P.wsK = NR;
+    if (gather || copy) {
+        grow(P.Xp, (size_t)P.npad * NR);
+        grow(P.Wp, (size_t)P.npad * NR);
     }
     for (uint32_t s0 = 0; s0 < k; s0 += NR) {
         const int kk = (int)std::min<uint32_t>(NR, k - s0);

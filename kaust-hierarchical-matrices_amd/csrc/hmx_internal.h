@@ -107,6 +107,16 @@ struct DBuf {
     size_t bytes() const { return n * sizeof(T); }
 };
 
+// Grows a workspace to n elements; true when it was allocated.  The buffer's
+// own size is the only record of it: a failed allocation leaves it empty, and
+// the next call, of whatever size, allocates again.
+template <class T>
+bool grow(DBuf<T>& b, size_t n) {
+    if (b.n >= n) return false;
+    b.alloc(n);
+    return true;
+}
+
 struct Context {
     hipStream_t stream = nullptr;
     int device = 0;
@@ -164,7 +174,6 @@ struct GradPlan {
     int64_t npad = 0;
     DBuf<int32_t> gmap;       // partial leaves: padded position -> vector index
     DBuf<double> Xp, Wp;      // padded copies of x and dY (partial leaves, unaligned vectors)
-    uint32_t wsK = 0;
     bool built = false;
 };
 
@@ -260,7 +269,6 @@ struct MatvecPlan {
     DBuf<int32_t> gmap;            // padded position -> vector index, -1 for padding
     // per-call workspaces (grown on demand)
     DBuf<double> zpart, z, Xp;
-    uint32_t wsK = 0;
 };
 
 // ---- multi right-hand-side (MFMA) matvec -----------------------------------
@@ -311,7 +319,6 @@ struct MfGroup {
                                    // 2 V, U and z (both phases)
     int64_t vLoOff = 0, uLoOff = 0; // split: the lo copies' offsets from the hi copies (FP16 elements)
     DBuf<unsigned char> zpart, zt; // workspaces
-    size_t wsNR = 0;               // pass width the workspaces are sized for
     int ztNR = 0;                  // pass width whose z padding columns were last cleared
 };
 
@@ -353,7 +360,6 @@ struct MfPlan {
     DBuf<double> origin;           // nearOtf: each leaf's first point, FP64 (x, y, z, w)
     float nlog2e = 0.f;            // -log2(e) / correlation length (nearOtf)
     DBuf<float> xscale, xpart;     // per right-hand-side scale and its per-slice partial maxima
-    size_t x16n = 0;
     float loMul = 1.f;             // 2^-E: FP16 z holds V^T x scaled by 2^E (mixed)
     float hiMul = 1.f;             // 2^(E - Ea): a split FP32 group's z holds V^T x scaled by 2^Ea
     // selection statistics (mixed)

@@ -424,7 +424,6 @@ void upload_plan(Context& c, MatvecPlan& P, const PlanHost& H) {
     }
     P.bytes = H.lowRankBytes + 8ull * (uint64_t)(S + P.numNear) * b * b;
     P.lowRankBytes = H.lowRankBytes;
-    P.wsK = 0;  // workspaces are sized for the previous plan
     HMX_HIP(hipStreamSynchronize(c.stream));
 }
 
@@ -500,12 +499,10 @@ static void run_phases(Context& c, const MatvecPlan& P, const MvWork& W, int b, 
 // Workspaces for passes of up to K right-hand sides.  Returns true when they
 // were (re)allocated: launch sequences captured before point at the old ones.
 bool ensure_matvec_ws(MatvecPlan& P, uint32_t K) {
-    if (P.wsK >= K) return false;
-    P.zpart.alloc((size_t)std::max<int64_t>(1, P.numPart) * K);
-    P.z.alloc((size_t)std::max<int64_t>(1, P.numCols) * K);
-    if (P.gather) P.Xp.alloc((size_t)P.npad * K);
-    P.wsK = K;
-    return true;
+    bool changed = grow(P.zpart, (size_t)std::max<int64_t>(1, P.numPart) * K);
+    changed = grow(P.z, (size_t)std::max<int64_t>(1, P.numCols) * K) || changed;
+    if (P.gather) changed = grow(P.Xp, (size_t)P.npad * K) || changed;
+    return changed;
 }
 
 // K = kernel width (1, 4, 8 or 16); k (a multiple of K) right-hand sides in

@@ -1967,13 +1967,11 @@ void reduce_group(Context& c, MfGroup& G, int NR, const float* rhsScale = nullpt
 // Returns true when a workspace was allocated or cleared (launch sequences
 // captured before then point at memory in another state).
 bool ensure_ws(Context& c, MfGroup& G, int NR, size_t accBytes) {
-    bool changed = false;
-    if (G.wsNR < (size_t)NR) {
-        G.zpart.alloc((size_t)std::max<int64_t>(1, G.numPart) * NR * accBytes);
-        G.zt.alloc((size_t)std::max<int64_t>(1, G.numColsPad) * NR * tsize(G.type));
-        G.wsNR = NR;
+    bool changed = grow(G.zpart, (size_t)std::max<int64_t>(1, G.numPart) * NR * accBytes);
+    const size_t zBytes = (size_t)std::max<int64_t>(1, G.numColsPad) * NR * tsize(G.type);
+    if (G.zt.n < zBytes) {
         G.ztNR = 0;
-        changed = true;
+        grow(G.zt, zBytes);
     }
     if (G.ztNR != NR) {
         HMX_HIP(hipMemsetAsync(G.zt.p, 0, G.zt.bytes(), c.stream));
@@ -2036,8 +2034,8 @@ void phase1(Context& c, MfGroup& G, const T* Xb, int sh, int kvalid, int xcdChun
 }
 
 // the lo half of a split group's FP16 z (MfGroup::split == 2): after the hi
-// half, whose size is fixed by the widest pass the workspace was made for
-int64_t split_zlo(const MfGroup& G) { return std::max<int64_t>(1, G.numColsPad) * (int64_t)G.wsNR; }
+// half, in the middle of a buffer made for the widest pass so far
+int64_t split_zlo(const MfGroup& G) { return (int64_t)(G.zt.n / (2 * sizeof(_Float16))); }
 
 // phase 1 of a mixed plan's FP32 group held as FP16 hi + lo (MfGroup::split):
 // TZ = float writes FP32 z in true units (rhsScale), TZ = _Float16 FP16 hi +
@@ -2209,8 +2207,8 @@ void finish_timing(Events& ev, float* acc) {
 bool ensure_fp64_ws(Context& c, MfPlan& P, int NR) {
     bool changed = ensure_ws(c, P.g[0], NR, sizeof(double));
     const size_t xb = (size_t)P.npad * NR * sizeof(double);
-    if (P.Xb.n < xb) { P.Xb.alloc(xb); changed = true; }
-    if (P.gather && P.Yp.n < xb) { P.Yp.alloc(xb); changed = true; }
+    changed = grow(P.Xb, xb) || changed;
+    if (P.gather) changed = grow(P.Yp, xb) || changed;
     return changed;
 }
 
@@ -2494,17 +2492,13 @@ void hmatrix_make_mixed(Context& c, HMatrix& h, double target) {
 bool ensure_mixed_ws(Context& c, MfPlan& P, int NR) {
     bool changed = ensure_ws(c, P.g[0], NR, sizeof(float));
     changed = ensure_ws(c, P.g[1], NR, sizeof(float)) || changed;
-    if (P.x16n < (size_t)P.npad * NR) {
-        P.X16.alloc((size_t)P.npad * NR);
-        if (P.nearOtf || P.g[0].split) P.X16lo.alloc((size_t)P.npad * NR);
-        P.Xb.alloc((size_t)P.npad * NR * sizeof(float));
-        if (P.gather) P.Yp.alloc((size_t)P.npad * NR * sizeof(float));
-        P.x16n = (size_t)P.npad * NR;
-        changed = true;
-    }
-    if (P.xscale.n < (size_t)NR) {
-        P.xscale.alloc(NR);
-        P.xpart.alloc((size_t)NR * kXSlices);
+    const size_t xn = (size_t)P.npad * NR;
+    changed = grow(P.X16, xn) || changed;
+    if (P.nearOtf || P.g[0].split) changed = grow(P.X16lo, xn) || changed;
+    changed = grow(P.Xb, xn * sizeof(float)) || changed;
+    if (P.gather) changed = grow(P.Yp, xn * sizeof(float)) || changed;
+    changed = grow(P.xpart, (size_t)NR * kXSlices) || changed;
+    if (grow(P.xscale, NR)) {
         // scales past a call's width are never set; the split FP32 group's
         // reduction multiplies its (zero) partials of those columns by them
         HMX_HIP(hipMemsetAsync(P.xscale.p, 0, P.xscale.bytes(), c.stream));

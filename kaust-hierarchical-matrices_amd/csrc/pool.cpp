@@ -48,12 +48,17 @@ struct Place {
 
 constexpr int kDevices = 64;
 std::mutex g_mu;
-Pool g_pool[kDevices];
-// never destroyed: handles may be freed while the process ends
-std::unordered_map<void*, Place>& places() {
-    static auto* m = new std::unordered_map<void*, Place>();
-    return *m;
+struct State {
+    Pool pool[kDevices];
+    std::unordered_map<void*, Place> places;
+};
+// never destroyed: handles and contexts may go while the process ends
+State& state() {
+    static auto* s = new State();
+    return *s;
 }
+Pool& pool(int device) { return state().pool[device]; }
+std::unordered_map<void*, Place>& places() { return state().places; }
 uint64_t g_seq = 1;
 int g_contexts = 0;
 
@@ -109,7 +114,7 @@ void* pool_alloc(size_t bytes) {
     int dev = 0;
     HMX_HIP(hipGetDevice(&dev));
     HMX_CHECK(dev >= 0 && dev < kDevices, HMX_EUNSUPPORTED, "device index beyond the pool table");
-    Pool& P = g_pool[dev];
+    Pool& P = pool(dev);
     size_t want = rounded(bytes);
     {
         std::unique_lock<std::mutex> lk(g_mu);
@@ -153,7 +158,7 @@ void pool_free(void* p) {
     auto it = places().find(p);
     if (it == places().end()) return;
     const Place at = it->second;
-    Pool& P = g_pool[at.device];
+    Pool& P = pool(at.device);
     if (g_contexts == 0 || at.bytes > P.bound) {
         places().erase(it);
         lk.unlock();
@@ -176,7 +181,7 @@ size_t pool_held_bytes() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return 0;
     std::lock_guard<std::mutex> lk(g_mu);
-    return g_pool[dev].bytes;
+    return pool(dev).bytes;
 }
 
 void pool_context_created() {
@@ -187,7 +192,7 @@ void pool_context_created() {
 void pool_context_destroyed() {
     std::lock_guard<std::mutex> lk(g_mu);
     if (--g_contexts > 0) return;
-    for (Pool& P : g_pool) flush(P);
+    for (Pool& P : state().pool) flush(P);
 }
 
 }  // namespace hmx

@@ -96,6 +96,14 @@ typedef struct hmx_hmatrix hmx_hmatrix;
    (src/main.cu:62). */
 hmx_status hmx_create(hmx_context** ctx, void* stream);
 hmx_status hmx_destroy(hmx_context* ctx);
+/* Device memory the library frees is held for its next allocations: at most
+   1/16 of the device's memory and 1/8 of what is free on it.  It goes back to
+   the driver when an allocation of the library finds no other memory, with
+   the last context, and with hmx_memory_release: for a caller whose own
+   allocation failed or is about to need the room.  Both calls are about the
+   current device. */
+hmx_status hmx_memory_held(hmx_context* ctx, uint64_t* bytes);
+hmx_status hmx_memory_release(hmx_context* ctx);
 const char* hmx_last_error(const hmx_context* ctx);
 /* parseArgs defaults, src/config.h:119-127 */
 void hmx_config_default(hmx_config* cfg);

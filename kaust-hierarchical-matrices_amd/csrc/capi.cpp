@@ -104,6 +104,19 @@ hmx_status hmx_destroy(hmx_context* ctx) {
     return HMX_OK;
 }
 
+hmx_status hmx_memory_held(hmx_context* ctx, uint64_t* bytes) {
+    if (!ctx) return HMX_EINVAL;
+    return guard(ctx, [&] {
+        NEED(bytes);
+        *bytes = pool_held_bytes();
+    });
+}
+
+hmx_status hmx_memory_release(hmx_context* ctx) {
+    if (!ctx) return HMX_EINVAL;
+    return guard(ctx, [&] { pool_release(); });
+}
+
 const char* hmx_last_error(const hmx_context* ctx) { return ctx ? ctx->last_error.c_str() : g_noctx_error.c_str(); }
 
 void hmx_config_default(hmx_config* cfg) {

@@ -51,6 +51,7 @@ inline void alloc_fault_point() {
 void* pool_alloc(size_t bytes);
 void pool_free(void* p);
 size_t pool_held_bytes();  // held on the current device
+void pool_release();       // gives back what is held on the current device
 void pool_context_created();
 void pool_context_destroyed();  // the last one gives everything held back
 

@@ -5,11 +5,16 @@
 // 3D build at N = 65536).  Blocks the library frees are therefore kept for
 // its next allocations of about their size:
 //
-//   * bounded: at most 1/16 of the device's memory is held (18 GB of 288);
-//     the blocks held longest go back to the driver first, and blocks above
-//     that bound are never held;
+//   * bounded: at most 1/16 of the device's memory is held (18 GB of 288; the
+//     3D build at N = 65536 leaves 12 GB, and takes 70 ms, with 1/64 75, with
+//     1/256 77, with nothing held 80; the TLR build 21, 21, 31 and 32 ms), and
+//     at most 1/8 of what is free on it (asked once per 1/1024 of the device
+//     that comes back: 4.7 us), so that on a full card little is kept from
+//     other allocators; the blocks held longest go back to the driver first,
+//     and blocks above the bound are never held;
 //   * given back: when the device has no memory left for an allocation of
-//     the library, and when the last context is destroyed;
+//     the library, when the caller asks (hmx_memory_release), and when the
+//     last context is destroyed;
 //   * as safe as hipFree with several streams and threads: a freed block is
 //     handed out again only after a wait for the device that followed its
 //     release, so no kernel or copy of any stream still uses it (hipFree made
@@ -18,6 +23,7 @@
 //     capture is refused where hipMalloc is, and neither disturbs a capture of
 //     another thread;
 //   * per device: a block returns to the device that it came from.
+#include <algorithm>
 #include <cstdint>
 #include <list>
 #include <mutex>
@@ -38,6 +44,8 @@ struct Pool {
     std::list<Held> held;  // in the order of release
     size_t bytes = 0;      // sum over held
     size_t bound = 0;      // most bytes held (0: not asked yet)
+    size_t limit = 0;      // the same by the device's free memory, when last asked
+    size_t back = 0;       // bytes released since then
     uint64_t synced = 0;   // blocks released before this number may be handed out
 };
 
@@ -72,7 +80,9 @@ size_t rounded(size_t n) {
     return (n + q - 1) / q * q;
 }
 
-// takes out the smallest held block of bytes or up to a quarter more
+// takes out the smallest held block of bytes or up to a quarter more (exact
+// sizes only, or up to twice: the builds take the same time; a quarter wastes
+// less of a long-lived object's memory than twice)
 void* take(Pool& P, size_t bytes, bool syncedOnly) {
     auto best = P.held.end();
     for (auto it = P.held.begin(); it != P.held.end(); ++it)
@@ -121,7 +131,7 @@ void* pool_alloc(size_t bytes) {
         if (P.bound == 0) {
             size_t fr = 0, tot = 0;
             HMX_HIP(hipMemGetInfo(&fr, &tot));
-            P.bound = tot / 16;
+            P.bound = P.limit = tot / 16;
         }
         if (want > P.bound / 4) want = bytes;  // large blocks: no memory given away to rounding
         if (void* p = take(P, want, true)) return p;
@@ -167,14 +177,29 @@ void pool_free(void* p) {
     }
     P.held.push_back(Held{p, at.bytes, g_seq++});
     P.bytes += at.bytes;
+    P.back += at.bytes;
+    int dev = -1;
+    if (P.back >= P.bound / 64 && hipGetDevice(&dev) == hipSuccess && dev == at.device) {
+        size_t fr = 0, tot = 0;
+        P.back = 0;
+        P.limit = hipMemGetInfo(&fr, &tot) == hipSuccess ? std::min(P.bound, fr / 8) : P.bound;
+    }
     std::list<Held> out;  // the blocks held longest, until the bound holds
-    while (P.bytes > P.bound) {
+    while (P.bytes > P.limit) {
         P.bytes -= P.held.front().bytes;
         places().erase(P.held.front().p);
         out.splice(out.end(), P.held, P.held.begin());
     }
     lk.unlock();
     for (const Held& h : out) (void)hipFree(h.p);
+}
+
+void pool_release() {
+    int dev = 0;
+    HMX_HIP(hipGetDevice(&dev));
+    HMX_HIP(hipFree(nullptr));  // not inside a capture
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (dev >= 0 && dev < kDevices) flush(pool(dev));
 }
 
 size_t pool_held_bytes() {

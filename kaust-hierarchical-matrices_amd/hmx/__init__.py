@@ -63,6 +63,8 @@ _P = ctypes.POINTER
 _SIGS = [
     ("hmx_create", _i32, [_P(_vp), _vp]),
     ("hmx_destroy", _i32, [_vp]),
+    ("hmx_memory_held", _i32, [_vp, _P(_u64)]),
+    ("hmx_memory_release", _i32, [_vp]),
     ("hmx_last_error", ctypes.c_char_p, [_vp]),
     ("hmx_config_default", None, [_P(Config)]),
     ("hmx_version", ctypes.c_char_p, []),
@@ -195,6 +197,19 @@ class Context:
                 self.handle = None
         except Exception:  # interpreter shutdown
             pass
+
+
+def memory_held(ctx):
+    """Device bytes the library holds for its next allocations."""
+    b = _u64()
+    _check(lib().hmx_memory_held(ctx.handle, ctypes.byref(b)), ctx)
+    return b.value
+
+
+def memory_release(ctx):
+    """Gives the held device memory back (for other allocators of the process,
+    as torch.cuda.empty_cache does with torch's)."""
+    _check(lib().hmx_memory_release(ctx.handle), ctx)
 
 
 class _Obj:

@@ -1,6 +1,7 @@
 // Host check of the library's held device memory (csrc/pool.cpp) over a
 // stand-in HIP runtime: a device of 1 GiB whose memory is host memory.
 //   pool_check hold      bound, order of giving back, out of memory, last context
+//   pool_check share     a full device: little is held, and given back when asked
 //   pool_check wait      a block is handed out again only after a device wait
 //   pool_check capture   allocation is refused where hipMalloc is
 //   pool_check exit      a handle and its context that go after the library's statics
@@ -119,6 +120,34 @@ static void hold() {
     REQUIRE(pool_held_bytes() == 0 && g_used == 0);
 }
 
+static void share() {
+    pool_context_created();
+    // somebody else's memory: 104 MiB of the device are left
+    g_used += kTotal - 104 * MB;
+    std::vector<void*> p;
+    for (int i = 0; i < 10; ++i) p.push_back(pool_alloc(4 * MB));
+    for (void* q : p) {
+        pool_free(q);
+        REQUIRE(pool_held_bytes() <= (kTotal - g_used) / 8);
+    }
+    REQUIRE(pool_held_bytes() > 0 && pool_held_bytes() <= 13 * MB);
+    pool_release();
+    REQUIRE(pool_held_bytes() == 0 && g_used == kTotal - 104 * MB);
+    // in a capture nothing is given back, and nothing is lost
+    pool_free(pool_alloc(4 * MB));
+    g_capturing = true;
+    bool refused = false;
+    try {
+        pool_release();
+    } catch (const Error&) {
+        refused = true;
+    }
+    g_capturing = false;
+    REQUIRE(refused && pool_held_bytes() == 4 * MB);
+    pool_context_destroyed();
+    REQUIRE(g_used == kTotal - 104 * MB);
+}
+
 static void wait() {
     pool_context_created();
     void* a = pool_alloc(2 * MB);
@@ -183,6 +212,7 @@ static LateHandle g_late __attribute__((init_priority(101)));
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "hold")) hold();
+    else if (!std::strcmp(what, "share")) share();
     else if (!std::strcmp(what, "wait")) wait();
     else if (!std::strcmp(what, "capture")) capture();
     else if (!std::strcmp(what, "exit")) {

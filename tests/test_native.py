@@ -31,6 +31,6 @@ def test_a_failed_growth_is_not_recorded(tmp_path):
     assert "buffer check ok" in run(tmp_path, "buffer_check")
 
 
-@pytest.mark.parametrize("what", ["hold", "wait", "capture", "exit"])
+@pytest.mark.parametrize("what", ["hold", "share", "wait", "capture", "exit"])
 def test_held_device_memory(tmp_path, what):
     assert f"pool check {what} ok" in run(tmp_path, "pool_check", ["pool.cpp"], [what])

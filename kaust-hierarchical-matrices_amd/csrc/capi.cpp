@@ -713,11 +713,23 @@ hmx_status hmx_HMatrixVecMultTranspose(hmx_context* ctx, const hmx_hmatrix* h, u
     if (!ctx) return HMX_EINVAL;
     return guard(ctx, [&] {
         NEED(h);
-        // as the forward product: two or more right-hand sides on the matrix cores
-        if (vectorWidth >= 2)
-            hmatvec_multi(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, nullptr, 0, true);
-        else
-            hmatvec(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, true, nullptr, 0);
+        hmx_hmatrix& H = const_cast<hmx_hmatrix&>(*h);
+        // as the forward product: two or more right-hand sides on the matrix
+        // cores.  Their plan has dense blocks and z of its own beside the
+        // forward one's (N = 2^20 3D, 64 right-hand sides: 37 GB more);
+        // where the device has no memory for it, the streaming kernels.
+        if (vectorWidth >= 2 && !H.mf64T.noMemory) {
+            try {
+                hmatvec_multi(*ctx, H, vectorWidth, d_in, d_out, nullptr, 0, true);
+                return;
+            } catch (const Error& e) {
+                if (e.status != HMX_ENOMEM) throw;
+                (void)hipGetLastError();
+                H.mf64T = MfPlan();
+                H.mf64T.noMemory = true;
+            }
+        }
+        hmatvec(*ctx, H, vectorWidth, d_in, d_out, true, nullptr, 0);
     });
 }
 

@@ -361,6 +361,12 @@ struct MfPlan {
     DBuf<double> origin;           // nearOtf: each leaf's first point, FP64 (x, y, z, w)
     float nlog2e = 0.f;            // -log2(e) / correlation length (nearOtf)
     DBuf<float> xscale, xpart;     // per right-hand-side scale and its per-slice partial maxima
+    // 16-column blocks of the widest pass: fewer once the device had no memory
+    // for z and the vectors of 64 right-hand sides
+    int maxBlocks = 4;
+    // transposed plan: the device had no memory for it (the streaming kernels
+    // do the product)
+    bool noMemory = false;
     float loMul = 1.f;             // 2^-E: FP16 z holds V^T x scaled by 2^E (mixed)
     float hiMul = 1.f;             // 2^(E - Ea): a split FP32 group's z holds V^T x scaled by 2^Ea
     // selection statistics (mixed)
@@ -478,9 +484,10 @@ bool ensure_matvec_ws(MatvecPlan& P, uint32_t K);
 // Every pass reads all factors, so one of 32 beats two of 16 (N = 60000 3D:
 // FP64 1.53 against 2.41 ms, mixed 0.46 against 0.81), one of 48 three (2.04
 // against 3.63; 0.52 against 1.21) and one of 64 four even for 50 right-hand
-// sides (2.45 against 4.81; 0.57 against 1.61).
-inline int mf_pass_blocks(uint32_t k) {
-    const uint32_t passes = (k + 63) / 64;
+// sides (2.45 against 4.81; 0.57 against 1.61).  most: the widest the plan has
+// memory for (MfPlan::maxBlocks).
+inline int mf_pass_blocks(uint32_t k, int most = 4) {
+    const uint32_t widest = 16u * (uint32_t)most, passes = (k + widest - 1) / widest;
     return (int)(((k + passes - 1) / passes + 15) / 16);
 }
 // widest streaming-kernel pass (16, 8, 4 or 1 right-hand sides) for rem columns

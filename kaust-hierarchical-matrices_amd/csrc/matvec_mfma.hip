@@ -2203,19 +2203,52 @@ void finish_timing(Events& ev, float* acc) {
 
 }  // namespace
 
-// Workspaces of an FP64 plan for passes of NR right-hand sides
-bool ensure_fp64_ws(Context& c, MfPlan& P, int NR) {
-    bool changed = ensure_ws(c, P.g[0], NR, sizeof(double));
-    const size_t xb = (size_t)P.npad * NR * sizeof(double);
-    changed = grow(P.Xb, xb) || changed;
-    if (P.gather) changed = grow(P.Yp, xb) || changed;
-    return changed;
+// Calls ensure(NR) for the width of a call's passes.  Where the device has no
+// memory for it, the workspaces go back and the passes get narrower, down to
+// 16: z of 64 right-hand sides takes four times the memory of 16, and calls of
+// 17 to 63 ran in passes of 16 once.  The plan remembers.
+template <class F>
+bool fit_pass(MfPlan& P, uint32_t k, F&& ensure) {
+    bool dropped = false;
+    while (true) {
+        const int NB = mf_pass_blocks(k, P.maxBlocks);
+        try {
+            return ensure(16 * NB) || dropped;
+        } catch (const Error& e) {
+            if (e.status != HMX_ENOMEM || NB == 1) throw;
+            (void)hipGetLastError();
+        }
+        for (MfGroup& G : P.g) {
+            G.zpart.release();
+            G.zt.release();
+            G.ztNR = 0;
+        }
+        P.Xb.release();
+        P.Yp.release();
+        P.X16.release();
+        P.X16lo.release();
+        P.xscale.release();
+        P.xpart.release();
+        P.maxBlocks = NB - 1;
+        dropped = true;
+    }
+}
+
+// Workspaces of an FP64 plan for a call of k right-hand sides
+bool ensure_fp64_ws(Context& c, MfPlan& P, uint32_t k) {
+    return fit_pass(P, k, [&](int NR) {
+        bool changed = ensure_ws(c, P.g[0], NR, sizeof(double));
+        const size_t xb = (size_t)P.npad * NR * sizeof(double);
+        changed = grow(P.Xb, xb) || changed;
+        if (P.gather) changed = grow(P.Yp, xb) || changed;
+        return changed;
+    });
 }
 
 // Y = H X for k right-hand sides (ld = the plan's n) in passes of
 // mf_pass_blocks(k) * 16, the last pass padded with zero columns
 void run_fp64_plan(Context& c, MfPlan& P, uint32_t k, const double* d_in, double* d_out, Events& ev) {
-    const int NB = mf_pass_blocks(k), NR = 16 * NB;
+    const int NB = mf_pass_blocks(k, P.maxBlocks), NR = 16 * NB;
     for (uint32_t s0 = 0; s0 < k; s0 += NR) {
         const int kk = (int)std::min<uint32_t>(NR, k - s0);
         const double* X = d_in + (size_t)s0 * P.n;
@@ -2232,7 +2265,7 @@ void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, doubl
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = transpose ? h.mf64T : h.mf64;
     if (!P.built) build_fp64_plan_set(c, {&h}, P, transpose);
-    ensure_fp64_ws(c, P, 16 * mf_pass_blocks(k));
+    ensure_fp64_ws(c, P, k);
     Events ev;
     if (ms) ev.create();
     const int reps = ms ? std::max(1, iters) : 1;
@@ -2268,7 +2301,7 @@ bool batch_mf_prepare(Context& c, Batch& B, uint32_t k) {
         for (const HMatrix* h : B.hs) B.mfGen.push_back(h->factorGen);
         changed = true;
     }
-    return ensure_fp64_ws(c, B.mf, 16 * mf_pass_blocks(k)) || changed;
+    return ensure_fp64_ws(c, B.mf, k) || changed;
 }
 
 void batch_mf_run(Context& c, Batch& B, uint32_t k, const double* d_in, double* d_out) {
@@ -2487,24 +2520,26 @@ void hmatrix_make_mixed(Context& c, HMatrix& h, double target) {
     P.built = true;
 }
 
-// Workspaces of the mixed plan for passes of NR right-hand sides; true when
-// any was allocated or cleared
-bool ensure_mixed_ws(Context& c, MfPlan& P, int NR) {
-    bool changed = ensure_ws(c, P.g[0], NR, sizeof(float));
-    changed = ensure_ws(c, P.g[1], NR, sizeof(float)) || changed;
-    const size_t xn = (size_t)P.npad * NR;
-    changed = grow(P.X16, xn) || changed;
-    if (P.nearOtf || P.g[0].split) changed = grow(P.X16lo, xn) || changed;
-    changed = grow(P.Xb, xn * sizeof(float)) || changed;
-    if (P.gather) changed = grow(P.Yp, xn * sizeof(float)) || changed;
-    changed = grow(P.xpart, (size_t)NR * kXSlices) || changed;
-    if (grow(P.xscale, NR)) {
-        // scales past a call's width are never set; the split FP32 group's
-        // reduction multiplies its (zero) partials of those columns by them
-        HMX_HIP(hipMemsetAsync(P.xscale.p, 0, P.xscale.bytes(), c.stream));
-        changed = true;
-    }
-    return changed;
+// Workspaces of the mixed plan for a call of k right-hand sides; true when any
+// was allocated or cleared
+bool ensure_mixed_ws(Context& c, MfPlan& P, uint32_t k) {
+    return fit_pass(P, k, [&](int NR) {
+        bool changed = ensure_ws(c, P.g[0], NR, sizeof(float));
+        changed = ensure_ws(c, P.g[1], NR, sizeof(float)) || changed;
+        const size_t xn = (size_t)P.npad * NR;
+        changed = grow(P.X16, xn) || changed;
+        if (P.nearOtf || P.g[0].split) changed = grow(P.X16lo, xn) || changed;
+        changed = grow(P.Xb, xn * sizeof(float)) || changed;
+        if (P.gather) changed = grow(P.Yp, xn * sizeof(float)) || changed;
+        changed = grow(P.xpart, (size_t)NR * kXSlices) || changed;
+        if (grow(P.xscale, NR)) {
+            // scales past a call's width are never set; the split FP32 group's
+            // reduction multiplies its (zero) partials of those columns by them
+            HMX_HIP(hipMemsetAsync(P.xscale.p, 0, P.xscale.bytes(), c.stream));
+            changed = true;
+        }
+        return changed;
+    });
 }
 
 // Y = H X for any k >= 1 (FP32, ld n) in passes of mf_pass_blocks(k) * 16,
@@ -2514,9 +2549,8 @@ void hmatvec_mixed(Context& c, HMatrix& h, uint32_t k, const float* d_in, float*
     HMX_CHECK(k >= 1, HMX_EINVAL, "mixed matvec: vectorWidth must be >= 1");
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = h.mfMixed;
-    const int NB = mf_pass_blocks(k);
-    const int NR = 16 * NB;
-    ensure_mixed_ws(c, P, NR);
+    ensure_mixed_ws(c, P, k);
+    const int NB = mf_pass_blocks(k, P.maxBlocks), NR = 16 * NB;
     Events ev;
     if (ms) ev.create();
     const int reps = ms ? std::max(1, iters) : 1;

@@ -51,9 +51,9 @@ void batch_create(Context& c, const std::vector<HMatrix*>& hs, Batch& B) {
 // One right-hand side: the streaming kernels.  Two or more: the FP64 matrix
 // cores over the batch's block-diagonal operator (passes of 16 to 64, the
 // last padded with zero columns).  Plans and workspaces are made ready here,
-// never inside a capture; when any of them was rebuilt, reallocated or
-// cleared the batch's epoch moves on, and a graph captured in an earlier
-// epoch is captured again before its next replay.
+// never inside a capture; when any of them was rebuilt or reallocated the
+// batch's epoch moves on, and a graph captured in an earlier epoch is captured
+// again before its next replay.
 static void prepare(Context& c, Batch& B, uint32_t k) {
     bool changed = false;
     if (k >= 2) {

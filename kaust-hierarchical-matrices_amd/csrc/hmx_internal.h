@@ -320,7 +320,6 @@ struct MfGroup {
                                    // 2 V, U and z (both phases)
     int64_t vLoOff = 0, uLoOff = 0; // split: the lo copies' offsets from the hi copies (FP16 elements)
     DBuf<unsigned char> zpart, zt; // workspaces
-    int ztNR = 0;                  // pass width whose z padding columns were last cleared
 };
 
 // Leaf-level tile stored dense in a matrix-core plan (rank above b/2: the

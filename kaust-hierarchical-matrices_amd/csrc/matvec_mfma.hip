@@ -518,6 +518,8 @@ __global__ void __launch_bounds__(256) k_mf_reduce(int64_t nred, int64_t ldz, co
 // acc[rg][nb] += U[16rg.., cols] Z[cols, rhs 16nb..].  The operands of the
 // next 16*KL-column step (possibly of the next entry) load while the current
 // step's MFMAs run.  rowOff: the wave's first row inside the entries' U.
+// z past an entry's rank is nobody's (U is zero there, but 0 * NaN left by an
+// earlier call would not be): it is taken as zero.
 template <int RG, bool UCM, class T, int NB>
 __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1, const T* __restrict__ Z, int rowOff,
                                int lg, int lc, int kvalid, typename Mfma<T>::accv (&acc)[RG][NB]) {
@@ -576,7 +578,7 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
         // a wait names the step it needs and not all that is in flight.
         constexpr int P = NB > 1 ? 2 : (RG * sizeof(T) >= 32 ? 3 : kPipe);
         T pa[P][RG][VL], pb[P][NB][VL];
-        int left[P], ranks[P];  // columns from the step's first on: padded, present
+        int left[P], ranks[P];  // columns from the step's first on: padded (0: past the list), present
         int e = e0, c0 = 0;
         const MfEntry* pe = ents + e;
         const void* eu = pe->u;
@@ -636,13 +638,13 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
         while (left[0] > 0) {  // a round: its steps past the end multiply zeros
 #pragma unroll
             for (int d = 0; d < P; ++d) {
-                if (min(left[d], UCM ? ranks[d] : left[d]) < SS) {
-                    const bool in = VL * lg < left[d];
+                const int have = min(left[d], ranks[d]);
+                if (have < SS) {
 #pragma unroll
                     for (int q = 0; q < VL; ++q) {
-                        const bool inA = UCM ? VL * lg + q < ranks[d] : in;
+                        const bool in = VL * lg + q < have;
 #pragma unroll
-                        for (int rg = 0; rg < RG; ++rg) pa[d][rg][q] = inA ? pa[d][rg][q] : (T)0;
+                        for (int rg = 0; rg < RG; ++rg) pa[d][rg][q] = in ? pa[d][rg][q] : (T)0;
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb) pb[d][nb][q] = in ? pb[d][nb][q] : (T)0;
                     }
@@ -666,10 +668,12 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
         int e = e0, c0 = 0;
         MfEntry en = ents[e], nx = ents[min(e + 1, e1 - 1)];
         bool full[kPipe];
+        int have[kPipe];  // columns present from the step's first on
         auto fill = [&](int d) {
             full[d] = e < e1;
             if (full[d]) {
                 load(en, c0, pa[d], pb[d]);
+                have[d] = en.rank - c0;
                 c0 += SS;
                 if (c0 >= en.rpad) {
                     c0 = 0;
@@ -685,6 +689,9 @@ __device__ inline void lr_rows(const MfEntry* __restrict__ ents, int e0, int e1,
 #pragma unroll
             for (int d = 0; d < kPipe; ++d)
                 if (full[d]) {
+                    if (have[d] < SS)
+#pragma unroll
+                        for (int q = 0; q < VL; ++q) pb[d][0][q] = VL * lg + q < have[d] ? pb[d][0][q] : (T)0;
 #pragma unroll
                     for (int q = 0; q < VL / MX::KL; ++q)
 #pragma unroll
@@ -740,6 +747,12 @@ __device__ inline void lr_rows_split(const MfEntry* __restrict__ ents, int e0, i
                         vzero(bl[nb]);
                     }
                 }
+                if (cc + VL > en.rank)  // as in lr_rows
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int q = 0; q < VL; ++q)
+                            if (cc + q >= en.rank) bh[nb][q] = bl[nb][q] = (_Float16)0;
             } else {
 #pragma unroll
                 for (int rg = 0; rg < RG; ++rg) {
@@ -1960,25 +1973,13 @@ void reduce_group(Context& c, MfGroup& G, int NR, const float* rhsScale = nullpt
     HMX_LAUNCHED();
 }
 
-// Workspaces.  The padding columns of z (rank rounded up to 16) are never
-// written by the kernels and must hold zeros: U is zero there, but 0 * NaN
-// left by an earlier call would not be.  Their positions depend on NR
-// (zt_index), so z is cleared again whenever the pass width changes.
-// Returns true when a workspace was allocated or cleared (launch sequences
-// captured before then point at memory in another state).
-bool ensure_ws(Context& c, MfGroup& G, int NR, size_t accBytes) {
+// Workspaces.  The padding columns of z (rank rounded up to 16), whose places
+// depend on NR (zt_index), are never written, and phase 2 takes no notice of
+// them.  Returns true when a workspace was allocated (launch sequences
+// captured before then point at freed memory).
+bool ensure_ws(MfGroup& G, int NR, size_t accBytes) {
     bool changed = grow(G.zpart, (size_t)std::max<int64_t>(1, G.numPart) * NR * accBytes);
-    const size_t zBytes = (size_t)std::max<int64_t>(1, G.numColsPad) * NR * tsize(G.type);
-    if (G.zt.n < zBytes) {
-        G.ztNR = 0;
-        grow(G.zt, zBytes);
-    }
-    if (G.ztNR != NR) {
-        HMX_HIP(hipMemsetAsync(G.zt.p, 0, G.zt.bytes(), c.stream));
-        G.ztNR = NR;
-        changed = true;
-    }
-    return changed;
+    return grow(G.zt, (size_t)std::max<int64_t>(1, G.numColsPad) * NR * tsize(G.type)) || changed;
 }
 
 // workgroups per XCD chunk in phase 1 (0: hardware order)
@@ -2221,7 +2222,6 @@ bool fit_pass(MfPlan& P, uint32_t k, F&& ensure) {
         for (MfGroup& G : P.g) {
             G.zpart.release();
             G.zt.release();
-            G.ztNR = 0;
         }
         P.Xb.release();
         P.Yp.release();
@@ -2235,9 +2235,9 @@ bool fit_pass(MfPlan& P, uint32_t k, F&& ensure) {
 }
 
 // Workspaces of an FP64 plan for a call of k right-hand sides
-bool ensure_fp64_ws(Context& c, MfPlan& P, uint32_t k) {
+bool ensure_fp64_ws(MfPlan& P, uint32_t k) {
     return fit_pass(P, k, [&](int NR) {
-        bool changed = ensure_ws(c, P.g[0], NR, sizeof(double));
+        bool changed = ensure_ws(P.g[0], NR, sizeof(double));
         const size_t xb = (size_t)P.npad * NR * sizeof(double);
         changed = grow(P.Xb, xb) || changed;
         if (P.gather) changed = grow(P.Yp, xb) || changed;
@@ -2265,7 +2265,7 @@ void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, doubl
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = transpose ? h.mf64T : h.mf64;
     if (!P.built) build_fp64_plan_set(c, {&h}, P, transpose);
-    ensure_fp64_ws(c, P, k);
+    ensure_fp64_ws(P, k);
     Events ev;
     if (ms) ev.create();
     const int reps = ms ? std::max(1, iters) : 1;
@@ -2287,7 +2287,7 @@ bool batch_mf_stale(const Batch& B) {
 
 // the FP64 plan of a batch, rebuilt when an instance's factors were
 // overwritten since (the plan may hold copies of them); true when the plan
-// was rebuilt or a workspace allocated or cleared
+// was rebuilt or a workspace allocated
 bool batch_mf_prepare(Context& c, Batch& B, uint32_t k) {
     bool changed = false;
     if (batch_mf_stale(B)) {
@@ -2301,7 +2301,7 @@ bool batch_mf_prepare(Context& c, Batch& B, uint32_t k) {
         for (const HMatrix* h : B.hs) B.mfGen.push_back(h->factorGen);
         changed = true;
     }
-    return ensure_fp64_ws(c, B.mf, k) || changed;
+    return ensure_fp64_ws(B.mf, k) || changed;
 }
 
 void batch_mf_run(Context& c, Batch& B, uint32_t k, const double* d_in, double* d_out) {
@@ -2524,8 +2524,8 @@ void hmatrix_make_mixed(Context& c, HMatrix& h, double target) {
 // was allocated or cleared
 bool ensure_mixed_ws(Context& c, MfPlan& P, uint32_t k) {
     return fit_pass(P, k, [&](int NR) {
-        bool changed = ensure_ws(c, P.g[0], NR, sizeof(float));
-        changed = ensure_ws(c, P.g[1], NR, sizeof(float)) || changed;
+        bool changed = ensure_ws(P.g[0], NR, sizeof(float));
+        changed = ensure_ws(P.g[1], NR, sizeof(float)) || changed;
         const size_t xn = (size_t)P.npad * NR;
         changed = grow(P.X16, xn) || changed;
         if (P.nearOtf || P.g[0].split) changed = grow(P.X16lo, xn) || changed;

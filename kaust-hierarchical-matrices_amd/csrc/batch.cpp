@@ -59,7 +59,9 @@ static void prepare(Context& c, Batch& B, uint32_t k) {
     if (k >= 2) {
         changed = batch_mf_prepare(c, B, k);
     } else {
-        if (p_stale(B)) {  // an instance's factors were overwritten: its dense blocks are stale
+        // an instance's factors were overwritten (its dense blocks are stale),
+        // or a rebuild ran out of memory half way
+        if (!B.P.built || p_stale(B)) {
             build_batch_plan(c, B.hs, B.P.chunk, B.P, B.diag);
             note_gens(B);
             changed = true;

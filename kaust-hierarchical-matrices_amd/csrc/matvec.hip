@@ -590,6 +590,7 @@ void hmatvec(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_o
 // vecBase_i = sum of the previous instances' n inside every right-hand side.
 void build_batch_plan(Context& c, const std::vector<HMatrix*>& hs, int chunk, MatvecPlan& P, DBuf<double>& diag) {
     HMX_CHECK(!hs.empty(), HMX_EINVAL, "empty batch");
+    P.built = false;
     const int b = (int)hs[0]->b;
     PlanHost B;
     B.b = b;

@@ -107,9 +107,10 @@ __global__ void __launch_bounds__(256) k_bbox_partial(uint32_t d, const double4*
     __shared__ double smin[4][3], smax[4][3];
     const int4 ch = chunks[blockIdx.x];
     double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+    const int cnt = ch.y - ch.x;  // positions reach 2^31 - 1: only offsets are stepped
 #pragma unroll 4
-    for (int i = ch.x + threadIdx.x; i < ch.y; i += 256) {
-        const double4 q = P4[perm[i]];
+    for (int o = threadIdx.x; o < cnt; o += 256) {
+        const double4 q = P4[perm[ch.x + o]];
         const double v[3] = {q.x, q.y, q.z};
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -199,8 +200,10 @@ __global__ void __launch_bounds__(256) k_radix_hist(KT* __restrict__ keys, const
     __syncthreads();
     const int4 ch = chunks[blockIdx.x];
     const uint32_t* rk = GATHER ? rank + (size_t)splitDim[ch.z] * n : nullptr;
+    const int size = ch.y - ch.x;
 #pragma unroll 4
-    for (int i = ch.x + threadIdx.x; i < ch.y; i += 256) {
+    for (int o = threadIdx.x; o < size; o += 256) {
+        const int i = ch.x + o;
         KT k;
         if constexpr (GATHER) {
             k = rk[perm[i]];
@@ -286,17 +289,17 @@ __global__ void __launch_bounds__(256) k_radix_scatter(const KT* __restrict__ ke
     int32_t rk[RD], dg[RD], val[RD];
     KT key[RD];
     const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+    const int size = ch.y - ch.x;
 #pragma unroll
     for (int r = 0; r < RD; ++r) {
-        const int i = ch.x + w * per + r * 64 + lane;
-        const bool valid = i < ch.y;
-        key[r] = valid ? keys[i] : (KT)0;
-        val[r] = valid ? vin[i] : 0;
+        const int o = w * per + r * 64 + lane;
+        const bool valid = o < size;
+        key[r] = valid ? keys[ch.x + o] : (KT)0;
+        val[r] = valid ? vin[ch.x + o] : 0;
     }
 #pragma unroll
     for (int r = 0; r < RD; ++r) {
-        const int i = ch.x + w * per + r * 64 + lane;
-        const bool valid = i < ch.y;
+        const bool valid = w * per + r * 64 + lane < size;
         const int d = (int)(key[r] >> shift) & mask;
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -495,7 +498,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_kd_small(int64_t n, const dou
 __global__ void __launch_bounds__(256) k_copy_segments(const int4* __restrict__ chunks, const int32_t* __restrict__ src,
                                                        int32_t* __restrict__ dst) {
     const int4 ch = chunks[blockIdx.x];
-    for (int i = ch.x + threadIdx.x; i < ch.y; i += 256) dst[i] = src[i];
+    for (int o = threadIdx.x; o < ch.y - ch.x; o += 256) dst[ch.x + o] = src[ch.x + o];
 }
 
 // the forest's points side by side: Pc[j * ntot + base_k + i] = p_k[j * n_k + i]

@@ -447,6 +447,11 @@ hmx_status hmx_batch_free(hmx_batch* batch);
 void hmx_debug_set_alloc_fault(int64_t failAt);
 int64_t hmx_debug_alloc_count(void);
 int64_t hmx_debug_live_bytes(void);
+/* The matrix-core products of an H-matrix give a wave 16 columns of an item
+   and 16 rows of a leaf in small plans, 64 columns and the whole leaf
+   otherwise, with equal results.  split: 1 always the former, 0 never, -1 by
+   size (the default). */
+hmx_status hmx_debug_set_wave_split(hmx_hmatrix* h, int32_t split);
 
 #ifdef __cplusplus
 }

@@ -798,6 +798,12 @@ hmx_status hmx_hmatrix_set_plan_options(hmx_hmatrix* h, int32_t denseNear, int32
     return HMX_OK;
 }
 
+hmx_status hmx_debug_set_wave_split(hmx_hmatrix* h, int32_t split) {
+    if (!h || split < -1 || split > 1) return HMX_EINVAL;
+    h->planSplit = split;
+    return HMX_OK;
+}
+
 hmx_status hmx_hmatrix_set_fp64_layout(hmx_hmatrix* h, int32_t layout) {
     if (!h || layout < 0 || layout > 2) return HMX_EINVAL;
     h->planFp64Layout = layout;

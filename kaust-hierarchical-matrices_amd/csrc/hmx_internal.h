@@ -366,6 +366,7 @@ struct MfPlan {
     // transposed plan: the device had no memory for it (the streaming kernels
     // do the product)
     bool noMemory = false;
+    int split = -1;                // HMatrix::planSplit
     float loMul = 1.f;             // 2^-E: FP16 z holds V^T x scaled by 2^E (mixed)
     float hiMul = 1.f;             // 2^(E - Ea): a split FP32 group's z holds V^T x scaled by 2^Ea
     // selection statistics (mixed)
@@ -388,6 +389,7 @@ struct HMatrix {
     MfPlan mf64, mf64T, mfMixed;
     // matrix-core plan choices (hmx_hmatrix_set_plan_options)
     int planDenseNear = 1;   // leaf-level tiles of rank > b/2 as dense blocks
+    int planSplit = -1;      // test hook: more waves per item and leaf always (1), never (0), by size (-1)
     int planDirectZ = 1;     // phase 1 stores whole-column z itself (else partials + reduce)
     int planLocality = 1;    // phase-1 items ordered by right-hand-side block
     int planFp64Layout = 0;  // FP64 plan factors: 0 copy when it fits in half the free memory, 1 in place, 2 copy

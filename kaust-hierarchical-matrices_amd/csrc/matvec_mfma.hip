@@ -2001,8 +2001,8 @@ int phase1_chunk() {
 // 228.  With enough waves the shared operands (right-hand sides, z) read more
 // often make it slower: N = 65536 2D (9200 items, 2048 leaves) phase 1 132 ->
 // 138, phase 2 141 -> 158 us; 60000 3D (1024 leaves of 64 rows) 648 -> 690.
-bool split_items(const MfGroup& G) { return G.numItems < 4096; }
-bool split_leaves(int S) { return S < 1024; }
+bool split_items(const MfPlan& P, const MfGroup& G) { return P.split < 0 ? G.numItems < 4096 : P.split > 0; }
+bool split_leaves(const MfPlan& P) { return P.split < 0 ? P.S < 1024 : P.split > 0; }
 
 // Workgroups of phase 2 (x) for so many waves, and workgroups per XCD chunk
 // (y).  Passes of 16 right-hand sides: chunks of 8 are dealt to the XCDs in
@@ -2042,13 +2042,12 @@ int64_t split_zlo(const MfGroup& G) { return (int64_t)(G.zt.n / (2 * sizeof(_Flo
 // TZ = float writes FP32 z in true units (rhsScale), TZ = _Float16 FP16 hi +
 // lo z in right-hand-side units
 template <int NB, class TZ>
-void phase1_split(Context& c, MfGroup& G, const _Float16* Xh, const _Float16* Xl, int sh, int kvalid,
+void phase1_split(Context& c, MfGroup& G, bool cols, const _Float16* Xh, const _Float16* Xl, int sh, int kvalid,
                   const float* rhsScale) {
     if (G.numItems == 0) return;
     HMX_CHECK(G.split == (sizeof(TZ) == 2 ? 2 : 1) && G.vfrag && G.colScaleV.n && Xl, HMX_ESTATE,
               "split phase 1: plan not built for it");
     const int chunk = phase1_chunk();
-    const bool cols = split_items(G);
     unsigned blocks = (unsigned)(((int64_t)G.numItems * (cols ? kMfCols / 16 : 1) + 3) / 4);
     if (chunk > 0) blocks = (blocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
     auto k1 = cols ? k_mf_phase1<_Float16, 1, NB, true, true, TZ> : k_mf_phase1<_Float16, 4, NB, true, true, TZ>;
@@ -2087,7 +2086,7 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
     k_x_blocked<double, double><<<(unsigned)((tot + 255) / 256), 256, 0, c.stream>>>(
         tot, P.npad, NR, sh, X, ldx, kk, P.gather ? P.gmap.p : nullptr, nullptr, (double*)P.Xb.p);
     HMX_LAUNCHED();
-    if (split_items(G)) phase1<double, 1, NB>(c, G, Xb, sh, kk, P.xcdChunk);
+    if (split_items(P, G)) phase1<double, 1, NB>(c, G, Xb, sh, kk, P.xcdChunk);
     else phase1<double, 4, NB>(c, G, Xb, sh, kk, P.xcdChunk);  // 4 column groups = the 64 columns of an item
     ev.rec(c, 1);
     reduce_group<double, double>(c, G, NR);
@@ -2097,7 +2096,7 @@ void run_fp64(Context& c, MfPlan& P, const double* X, int64_t ldx, int kk, doubl
     {
         const int* gp = G.grouped ? G.grpPtr.p : nullptr;
         const MfEntry* ge = G.grouped ? G.grpEntries.p : nullptr;
-        const bool split = split_leaves(P.S);
+        const bool split = split_leaves(P);
         const int2 pg = phase2_grid(P.S * (split ? P.b / 16 : 1), NB == 1);
         auto pick = [&](auto b, auto ucm) {
             constexpr int B = decltype(b)::value;
@@ -2144,10 +2143,10 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
                                                             P.X16.p, P.X16lo.n ? P.X16lo.p : nullptr);
     HMX_LAUNCHED();
     const float* Xb = (const float*)P.Xb.p;
-    if (Ghi.split == 2) phase1_split<NB, _Float16>(c, Ghi, P.X16.p, P.X16lo.p, sh16, kk, nullptr);
-    else if (Ghi.split == 1) phase1_split<NB, float>(c, Ghi, P.X16.p, P.X16lo.p, sh16, kk, P.xscale.p);
+    if (Ghi.split == 2) phase1_split<NB, _Float16>(c, Ghi, split_items(P, Ghi), P.X16.p, P.X16lo.p, sh16, kk, nullptr);
+    else if (Ghi.split == 1) phase1_split<NB, float>(c, Ghi, split_items(P, Ghi), P.X16.p, P.X16lo.p, sh16, kk, P.xscale.p);
     else phase1<float, 4, NB>(c, Ghi, Xb, sh32, kk);
-    if (split_items(Glo)) phase1<_Float16, 1, NB>(c, Glo, P.X16.p, sh16, kk);
+    if (split_items(P, Glo)) phase1<_Float16, 1, NB>(c, Glo, P.X16.p, sh16, kk);
     else phase1<_Float16, 4, NB>(c, Glo, P.X16.p, sh16, kk);
     ev.rec(c, 1);
     if (Ghi.split == 2) reduce_group<float, _Float16>(c, Ghi, NR, nullptr, split_zlo(Ghi));
@@ -2160,7 +2159,7 @@ void run_mixed(Context& c, MfPlan& P, const float* X, int64_t ldx, int kk, float
         const bool gr = Ghi.grouped && Glo.grouped;
         const bool spa = Ghi.split == 2;
         // a split group's z is FP16 hi + lo (the kernel's ZA), else FP32
-        const bool split = !spa && split_leaves(P.S);
+        const bool split = !spa && split_leaves(P);
         const int2 pg = phase2_grid(P.S * (split ? P.b / 16 : 1), NB == 1);
         auto launch = [&](auto k2, const auto* za) {
             k2<<<pg.x, 256, 0, c.stream>>>(
@@ -2265,6 +2264,7 @@ void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, doubl
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = transpose ? h.mf64T : h.mf64;
     if (!P.built) build_fp64_plan_set(c, {&h}, P, transpose);
+    P.split = h.planSplit;
     ensure_fp64_ws(P, k);
     Events ev;
     if (ms) ev.create();
@@ -2549,6 +2549,7 @@ void hmatvec_mixed(Context& c, HMatrix& h, uint32_t k, const float* d_in, float*
     HMX_CHECK(k >= 1, HMX_EINVAL, "mixed matvec: vectorWidth must be >= 1");
     HMX_CHECK(d_in && d_out && d_in != d_out, HMX_EINVAL, "bad vector pointers");
     MfPlan& P = h.mfMixed;
+    P.split = h.planSplit;
     ensure_mixed_ws(c, P, k);
     const int NB = mf_pass_blocks(k, P.maxBlocks), NR = 16 * NB;
     Events ev;

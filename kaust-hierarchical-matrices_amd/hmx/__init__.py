@@ -130,6 +130,7 @@ _SIGS = [
     ("hmx_debug_set_alloc_fault", None, [_i64]),
     ("hmx_debug_alloc_count", _i64, []),
     ("hmx_debug_live_bytes", _i64, []),
+    ("hmx_debug_set_wave_split", _i32, [_vp, _i32]),
 ]
 
 

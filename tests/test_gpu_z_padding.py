@@ -44,11 +44,13 @@ def product(pp, path, X, Y=None):
     return pp.matvec(X, Y, transpose=path == "transposed")
 
 
+@pytest.mark.parametrize("split", [0, 1], ids=["whole-leaves", "split-leaves"])
 @pytest.mark.parametrize("path,layout", PATHS)
 @pytest.mark.parametrize("k,other", [(40, 8), (8, 40), (64, 20), (20, 64), (48, 33)])
-def test_a_graph_replayed_after_other_widths(torch_cuda, setup, path, layout, k, other):
+def test_a_graph_replayed_after_other_widths(torch_cuda, setup, path, layout, k, other, split):
     torch = torch_cuda
     s, pp, X = setup
+    assert hmx.lib().hmx_debug_set_wave_split(pp.H.handle, split) == hmx.HMX_OK
     with torch.cuda.stream(s):
         if layout:
             pp.H.set_fp64_layout(layout)

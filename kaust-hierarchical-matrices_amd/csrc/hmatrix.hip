@@ -774,9 +774,13 @@ __global__ void __launch_bounds__(1024) k_lr_decide(LrLevel L) {
 // What is left is the latency of a round (DPP sums, one barrier), some 256
 // of them per block.  The sums are formed in k_lr_decide's order, bit for
 // bit: the last columns of a tile are residuals 1e-7 of what was sampled, so
-// another order would move them by 1e-9 and more.  N = 65536 3D build, the
-// levels of 4096 and 8192 rows (15 blocks): decisions 13.6 -> 4.6 ms, the
-// renormalisation below 6.5 -> 2.5, against the columns re-read from memory.
+// another order would move them by 1e-9 and more.  The fused steps are
+// written out for that: of p = y0 y0 + y1 y1 the compiler may round either
+// product by itself, and k_lr_decide's loop rounds the first.  N = 65536 3D
+// build, the levels of 4096 and 8192 rows (15 blocks): decisions 13.6 -> 4.6
+// ms, the renormalisation below 6.5 -> 2.5, against the columns re-read from
+// memory.  16384 rows (N = 262144 3D and N = 65536 2D, 26 blocks each): 2.2 ->
+// 0.60 ms a block, 1.1 -> 0.35, also with the 13 registers that spill there.
 template <int R>
 __global__ void __launch_bounds__(1024) k_lr_decide_t(LrLevel L) {
     __shared__ double red[32];
@@ -806,7 +810,7 @@ __global__ void __launch_bounds__(1024) k_lr_decide_t(LrLevel L) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 n[r] = Qb[(size_t)nx * m + tid + 1024 * r];
-                p += q[r] * y[r];
+                p = fma(q[r], y[r], p);
             }
             const double d = block_sum(p, red, parity);
 #pragma unroll
@@ -817,7 +821,7 @@ __global__ void __launch_bounds__(1024) k_lr_decide_t(LrLevel L) {
         }
         double p = 0.0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) p += y[r] * y[r];
+        for (int r = 0; r < R; ++r) p = fma(y[r], y[r], p);
         const double nu = sqrt(block_sum(p, red, parity));
         if (nu > tau) {
             if (na >= capleft) { capped = 1; break; }
@@ -857,7 +861,7 @@ __global__ void __launch_bounds__(1024) k_lr_renorm_t(LrLevel L) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 n[r] = Qb[(size_t)(a + 1) * m + tid + 1024 * r];
-                p += q[r] * y[r];
+                p = fma(q[r], y[r], p);
             }
             const double d = block_sum(p, red, parity);
 #pragma unroll
@@ -868,7 +872,7 @@ __global__ void __launch_bounds__(1024) k_lr_renorm_t(LrLevel L) {
         }
         double p = 0.0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) p += y[r] * y[r];
+        for (int r = 0; r < R; ++r) p = fma(y[r], y[r], p);
         const double nu = sqrt(block_sum(p, red, parity));
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -1233,6 +1237,7 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
     const auto tB = std::chrono::steady_clock::now();
     const unsigned rowBlocks = (unsigned)((m + 63) / 64);
     const unsigned wgThreads = m >= 4096 ? 1024u : 256u;
+    const bool inRegs = !std::getenv("HMX_ARA_RELOAD");  // set by the test of k_lr_decide_t's bits
     int kmax = 0, preStart = 0, preN = 0, sweeps = 0;
     int active = T;  // tiles still iterating (the count k_lr_commit reports)
     const int maxIters = (2 * maxRank + araR) / kB16 + 2;
@@ -1288,9 +1293,9 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         else if (m == 512) k_lr_decide_w<8><<<T, 64, 0, c.stream>>>(L);
         else if (m == 1024) k_lr_decide_b<4><<<T, 256, 0, c.stream>>>(L);
         else if (m == 2048) k_lr_decide_b<8><<<T, 256, 0, c.stream>>>(L);
-        else if (m == 4096) k_lr_decide_t<4><<<T, 1024, 0, c.stream>>>(L);
-        else if (m == 8192) k_lr_decide_t<8><<<T, 1024, 0, c.stream>>>(L);
-        else if (m == 16384) k_lr_decide_t<16><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 4096) k_lr_decide_t<4><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 8192) k_lr_decide_t<8><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 16384) k_lr_decide_t<16><<<T, 1024, 0, c.stream>>>(L);
         else k_lr_decide<<<T, wgThreads, 0, c.stream>>>(L);
         HMX_LAUNCHED();
         if (kmax > 0) {
@@ -1305,9 +1310,9 @@ static void compress_batch(Context& c, int araR, uint64_t seed, const LevelSourc
         else if (m == 512) k_lr_renorm_w<8><<<T, 64, 0, c.stream>>>(L);
         else if (m == 1024) k_lr_renorm_b<4><<<T, 256, 0, c.stream>>>(L);
         else if (m == 2048) k_lr_renorm_b<8><<<T, 256, 0, c.stream>>>(L);
-        else if (m == 4096) k_lr_renorm_t<4><<<T, 1024, 0, c.stream>>>(L);
-        else if (m == 8192) k_lr_renorm_t<8><<<T, 1024, 0, c.stream>>>(L);
-        else if (m == 16384) k_lr_renorm_t<16><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 4096) k_lr_renorm_t<4><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 8192) k_lr_renorm_t<8><<<T, 1024, 0, c.stream>>>(L);
+        else if (inRegs && m == 16384) k_lr_renorm_t<16><<<T, 1024, 0, c.stream>>>(L);
         else k_lr_renorm<<<T, wgThreads, 0, c.stream>>>(L);
         HMX_LAUNCHED();
         HMX_HIP(hipMemsetAsync(ws.flags.p, 0, 2 * sizeof(int), c.stream));

@@ -1007,8 +1007,12 @@ __device__ inline void near_otf(int leaf, int w, int row0, const float4* __restr
 // held as FP16 hi + lo (U, and z in right-hand-side units times 2^Ea) goes
 // first instead, its sum multiplied by hiMul = 2^(E - Ea) into the FP16
 // group's units.
+//
+// Mixed: two waves per SIMD asked for.  64 right-hand sides over 64-row leaves
+// take 265 registers with one and 239 with two, without a spill; phase 2 at N =
+// 262144 3D 1.45 -> 1.27 ms, at 2^20 6.3 -> 5.4.
 template <int BL, bool UCM, class TD, class TA, class TB, int NB, class TO, bool SPA = false, int RG = BL / 16>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPA || (NB == 1 && in_line<TA, NB>(RG)) ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TA) < 8 || (NB == 1 && in_line<TA, NB>(RG)) ? 2 : 1))) k_mf_phase2g(int S, int chunk, const int32_t* __restrict__ ptrA, const MfEntry* __restrict__ entA,
                                                     const int32_t* __restrict__ gptrA,
                                                     const MfEntry* __restrict__ gentA, const TA* __restrict__ ZA,
                                                     const int32_t* __restrict__ ptrB, const MfEntry* __restrict__ entB,

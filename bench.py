@@ -175,6 +175,8 @@ def main():
     torch.cuda.empty_cache()
     log(f"streaming-read ceiling {read_ceiling:.0f} GB/s; dominant kernel {achieved:.0f} GB/s")
     # measured FP64 arithmetic ceilings (register-only chains, 8 waves per SIMD)
+    # the rate of independent 16x16x4 chains, 8 waves per SIMD: a yardstick, which real kernels of other
+    # shapes and occupancies can pass
     mfma_ceiling = hmx.fp64_peak_probe(ctx, 0)
     valu_ceiling = hmx.fp64_peak_probe(ctx, 1)
     log(f"FP64 ceilings: matrix cores {mfma_ceiling:.1f} TFLOP/s, vector FMA {valu_ceiling:.1f} TFLOP/s")

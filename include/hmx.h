@@ -290,7 +290,9 @@ hmx_status hmx_HMatrixVecMultNoAlloc(hmx_context* ctx, const hmx_hmatrix* h, uin
                                      const double* d_in, double* d_out);
 /* out = H^T * in (no reference counterpart; the backward of HMatrixVecMult);
    any vectorWidth >= 1 and any n: one right-hand side on the streaming
-   kernels, two or more on the matrix cores as hmx_HMatrixVecMult. */
+   kernels, two or more on the matrix cores as hmx_HMatrixVecMult, with a plan
+   of their own (dense blocks and z once more; on the streaming kernels where
+   the device has no memory for it). */
 hmx_status hmx_HMatrixVecMultTranspose(hmx_context* ctx, const hmx_hmatrix* h, uint32_t vectorWidth,
                                        const double* d_in, double* d_out);
 /* Times the matvec kernels with hipEvents on the context stream over iters
@@ -301,8 +303,9 @@ hmx_status hmx_matvec_profile(hmx_context* ctx, const hmx_hmatrix* h, uint32_t v
 
 /* ---- many right-hand sides on the matrix cores ------------------------- */
 /* hmx_HMatrixVecMult with vectorWidth >= 2 runs on the FP64 matrix cores
-   (passes of 64 right-hand sides when vectorWidth is a multiple of 64, else
-   of 16, the last pass padded with zero columns).  Times the multi-RHS
+   (passes of 16, 32, 48 or 64 right-hand sides, the fewest, all of one width;
+   narrower where the device has no memory for their workspaces; the last
+   pass padded with zero columns).  Times the multi-RHS
    kernels like hmx_matvec_profile (ms[0] phase 1, ms[1] reduce, ms[2] phase
    2, ms[3] call) for vectorWidth 16 or 64; mixed != 0 times
    hmx_HMatrixVecMultMixed (in/out then point to float). */

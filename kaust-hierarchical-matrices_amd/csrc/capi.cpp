@@ -591,7 +591,14 @@ hmx_status hmx_HMatrixVecMult(hmx_context* ctx, const hmx_hmatrix* h, uint32_t v
         NEED(h);
         // two or more right-hand sides: the FP64 matrix cores (passes of 16
         // to 64, partial leaves through the padded space); one: the
-        // streaming kernels
+        // streaming kernels.  Matrix cores against streaming passes of 4 and
+        // 1, us, 2 / 3 / 4 right-hand sides: N = 1000 2D 20 / 21 / 21 against
+        // 21 / 32 / 19, 16384 3D 180 / 182 / 185 against 261 / 392 / 188, 65536
+        // 2D 206 / 206 / 207 against 306 / 459 / 240, 100000 3D 2164 / 2167 /
+        // 2172 against 3573 / 5359 / -.  Only around N = 4096 2D are the
+        // streaming kernels ahead for 2 and 4 (40 / 40 / 40 against 27 / 41 /
+        // 32): the line stays at two, the same for every size, so that a batch
+        // and its instances take one path.
         if (vectorWidth >= 2)
             hmatvec_multi(*ctx, const_cast<hmx_hmatrix&>(*h), vectorWidth, d_in, d_out, nullptr, 0);
         else

@@ -483,9 +483,9 @@ bool ensure_matvec_ws(MatvecPlan& P, uint32_t K);
 // 16-column blocks (1 to 4) per matrix-core pass of k right-hand sides: the
 // fewest passes of at most 64, all of one width (z's layout depends on it).
 // Every pass reads all factors, so one of 32 beats two of 16 (N = 60000 3D:
-// FP64 1.53 against 2.41 ms, mixed 0.46 against 0.81), one of 48 three (2.04
-// against 3.63; 0.52 against 1.21) and one of 64 four even for 50 right-hand
-// sides (2.45 against 4.81; 0.57 against 1.61).  most: the widest the plan has
+// FP64 1.19 against 1.99 ms, mixed 0.42 against 0.74), one of 48 three (1.47
+// against 2.98; 0.46 against 1.11) and one of 64 four even for 50 right-hand
+// sides (1.78 against 3.98; 0.51 against 1.48).  most: the widest the plan has
 // memory for (MfPlan::maxBlocks).
 inline int mf_pass_blocks(uint32_t k, int most = 4) {
     const uint32_t widest = 16u * (uint32_t)most, passes = (k + widest - 1) / widest;

@@ -1999,12 +1999,13 @@ int phase1_chunk() {
 // item instead of all 64, phase 2 a wave per 16 rows of a leaf instead of the
 // leaf.  A lone wave on a SIMD waits out every product (79 to 137 clocks per
 // FP64 16x16x4, nothing else to issue), so the chip's 1024 SIMDs need several
-// waves each; the same sums are formed in the same order either way.  16
-// right-hand sides, FP64 / mixed: N = 4096 2D 98 -> 58 / 66 -> 53 us, 16384 3D
-// 479 -> 244 / 237 -> 132; 64: 288 -> 171 / 98 -> 75, 1301 -> 730 / 351 ->
-// 228.  With enough waves the shared operands (right-hand sides, z) read more
-// often make it slower: N = 65536 2D (9200 items, 2048 leaves) phase 1 132 ->
-// 138, phase 2 141 -> 158 us; 60000 3D (1024 leaves of 64 rows) 648 -> 690.
+// waves each; the same sums are formed in the same order either way.  Calls,
+// FP64 / mixed: 16 right-hand sides N = 4096 2D 70 -> 44 / 57 -> 45 us, 16384
+// 3D 453 -> 219 / 221 -> 115; 64: 197 -> 95 / 87 -> 64, 895 -> 519 / 315 -> 195.
+// With enough waves the shared operands (right-hand sides, z) read more often
+// make it slower: N = 65536 2D (9200 items, 2048 leaves) 16 right-hand sides 232
+// -> 255 / 130 -> 123 us, 64: 480 -> 566 / 201 -> 220; 60000 3D (1024 leaves of
+// 64 rows) 996 -> 1121 / 378 -> 371, 64: 1791 -> 2412 / 533 -> 631.
 bool split_items(const MfPlan& P, const MfGroup& G) { return P.split < 0 ? G.numItems < 4096 : P.split > 0; }
 bool split_leaves(const MfPlan& P) { return P.split < 0 ? P.S < 1024 : P.split > 0; }
 
@@ -2261,7 +2262,7 @@ void run_fp64_plan(Context& c, MfPlan& P, uint32_t k, const double* d_in, double
 }
 
 // transpose: H^T, through a plan of its own (N = 65536 2D, 32 right-hand
-// sides: 0.37 ms; the streaming kernels, 16 wide, took 1.9)
+// sides: 0.30 ms; the streaming kernels, 16 wide, took 1.9)
 void hmatvec_multi(Context& c, HMatrix& h, uint32_t k, const double* d_in, double* d_out, float* ms, int iters,
                    bool transpose) {
     HMX_CHECK(k >= 1, HMX_EINVAL, "multi-RHS matvec: vectorWidth must be >= 1");

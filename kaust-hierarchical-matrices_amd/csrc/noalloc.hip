@@ -72,7 +72,7 @@ void hmatvec_noalloc(Context& c, const HMatrix& h, uint32_t k, const double* X, 
     const size_t nSlots = round_up((size_t)std::max<int64_t>(1, P.numPart + P.numCols - P.numSplits) * K);
     const size_t need = (nSlots + nZ + 2 * nPad) * sizeof(double);
     HMX_CHECK(need <= kScratchBytes, HMX_EINVAL,
-              "the no-allocation H-matvec needs " + std::to_string(need >> 20) + " MiB of scratch for passes of " +
+              "the no-allocation H-matvec counts " + std::to_string(need >> 20) + " MiB of scratch for passes of " +
                   std::to_string(K) + " right-hand sides of this H-matrix; its fixed array holds " +
                   std::to_string(kScratchBytes >> 20) + " MiB");
     double* s = static_cast<double*>(base);
